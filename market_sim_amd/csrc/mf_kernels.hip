@@ -15,6 +15,8 @@
 namespace mf {
 namespace {
 
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / kWave;
 
@@ -627,19 +629,132 @@ __device__ __forceinline__ float logit_at(const void* p, uint64_t i) {
                : static_cast<const float*>(p)[i];
 }
 
+// greedy_select: one workgroup of 1024 threads per row.  Bound: a row's bytes
+// through one compute unit (there is no scratch memory to merge workgroups
+// through: the reference's operator takes none), so what counts is the bytes
+// in flight: kSelBatch 16-byte words per thread (128 KB per compute unit).
+// Each thread keeps the first of its words that holds its best value (a word
+// is compared by its maximum, NaN ignored), and only the threads whose best
+// is the row's maximum look for the element.  A row may start anywhere: the
+// elements before its first and after its last whole word are scalars.
+// V = 49152 FP16: 8 rows 89.9 -> 4.4 us, 256 rows 89.0 -> 6.8 us (from one
+// 2-byte load per thread and iteration in a 256-thread workgroup); one row of
+// 128256: 6.8 us.
+constexpr int kSelThreads = 1024;
+constexpr uint32_t kSelBatch = 8;
+
+// A signalling NaN would come out of a maximum as a NaN: made quiet first.
+__device__ __forceinline__ half2_t quiet(uint32_t v) {
+  return __builtin_elementwise_canonicalize(__builtin_bit_cast(half2_t, v));
+}
+
+// The largest value of a 16-byte word, NaN only if all are.
 template <bool kHalf>
-__global__ __launch_bounds__(kThreads) void greedy_kernel(
-    const void* __restrict__ logits, uint32_t* __restrict__ tokens, uint32_t V) {
-  __shared__ Red sh;
-  const uint64_t base = static_cast<uint64_t>(blockIdx.x) * V;
-  Best best = best_identity();
-  for (uint32_t c = threadIdx.x; c < V; c += kThreads) {
-    best = best_of(best, best_leaf(logit_at<kHalf>(logits, base + c), c, c));
+__device__ __forceinline__ float word_max(const uint4& q) {
+  if constexpr (kHalf) {
+    const half2_t m = __builtin_elementwise_max(
+        __builtin_elementwise_max(quiet(q.x), quiet(q.y)),
+        __builtin_elementwise_max(quiet(q.z), quiet(q.w)));
+    return __builtin_fmaxf(static_cast<float>(m.x), static_cast<float>(m.y));
+  } else {
+    const float a = __builtin_fmaxf(__builtin_canonicalizef(as_float(q.x)),
+                                    __builtin_canonicalizef(as_float(q.y)));
+    const float b = __builtin_fmaxf(__builtin_canonicalizef(as_float(q.z)),
+                                    __builtin_canonicalizef(as_float(q.w)));
+    return __builtin_fmaxf(a, b);
   }
-  best = block_best(sh, best);
-  if (threadIdx.x == 0) {
+}
+
+// Element k of a 16-byte word.
+template <bool kHalf>
+__device__ __forceinline__ float word_element(const uint4& q, uint32_t k) {
+  const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+  if constexpr (kHalf) {
+    return half_to_float(static_cast<uint16_t>(w[k / 2u] >> (16u * (k % 2u))));
+  } else {
+    return as_float(w[k]);
+  }
+}
+
+template <bool kHalf>
+__global__ __launch_bounds__(kSelThreads) void greedy_kernel(
+    const void* __restrict__ logits, uint32_t* __restrict__ tokens, uint32_t V) {
+  constexpr uint32_t kSize = kHalf ? 2u : 4u;
+  constexpr uint32_t kPer = 16u / kSize;  // elements per word
+  constexpr int kSelWaves = kSelThreads / kWave;
+  __shared__ float red_f[kSelWaves];
+  __shared__ uint32_t red_t[kSelWaves];
+  const uint32_t tid = threadIdx.x;
+  const uint64_t base = static_cast<uint64_t>(blockIdx.x) * V;
+  const uintptr_t at = reinterpret_cast<uintptr_t>(logits) + base * kSize;
+  // elements before the first whole word (all of them if no word is aligned)
+  const uint32_t lead = static_cast<uint32_t>((0u - at) % 16u);
+  const uint32_t head = (lead % kSize != 0u || lead / kSize > V) ? V : lead / kSize;
+  const uint32_t words = (V - head) / kPer;
+  const uint32_t tail = head + words * kPer;  // the first element after the words
+  const uint4* row = reinterpret_cast<const uint4*>(at + static_cast<uintptr_t>(head) * kSize);
+
+  const float low = -__builtin_huge_valf();
+  float best = low;  // strictly greater wins: the first word of a thread's best value
+  uint32_t word = 0u;
+  uint4 hold{0u, 0u, 0u, 0u};
+  for (uint32_t q0 = tid; q0 < words; q0 += kSelThreads * kSelBatch) {
+    uint4 v[kSelBatch];
+#pragma unroll
+    for (uint32_t u = 0; u < kSelBatch; ++u) {  // past the end: the last word again
+      const uint32_t q = q0 + u * kSelThreads;
+      v[u] = row[q < words ? q : words - 1u];
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < kSelBatch; ++u) {
+      const uint32_t q = q0 + u * kSelThreads;
+      const float m = word_max<kHalf>(v[u]);
+      if (m > best) {
+        best = m;
+        word = q < words ? q : words - 1u;
+        hold = v[u];
+      }
+    }
+  }
+  float edge = low;  // the scalars of this thread, in ascending order
+  uint32_t edge_token = kInvalidToken;
+  for (uint64_t c = tid; c < head + (V - tail); c += kSelThreads) {
+    const uint32_t t = static_cast<uint32_t>(c < head ? c : tail + (c - head));
+    const float v = logit_at<kHalf>(logits, base + t);
+    if (v > edge) {
+      edge = v;
+      edge_token = t;
+    }
+  }
+  const float mine = wave_max(__builtin_fmaxf(best, edge));
+  if (tid % kWave == 0u) red_f[tid / kWave] = mine;
+  __syncthreads();
+  float top = red_f[0];
+#pragma unroll
+  for (int i = 1; i < kSelWaves; ++i) top = __builtin_fmaxf(top, red_f[i]);
+  uint32_t token = kInvalidToken;
+  if (top > low) {
+    if (edge == top) token = edge_token;
+    if (best == top) {
+#pragma unroll
+      for (int k = static_cast<int>(kPer) - 1; k >= 0; --k) {
+        const uint32_t t = head + word * kPer + static_cast<uint32_t>(k);
+        if (word_element<kHalf>(hold, static_cast<uint32_t>(k)) == top && t < token) token = t;
+      }
+    }
+  } else {  // nothing above -inf: the lowest -inf, or token 0 if all are NaN
+    for (uint64_t c = tid; c < V && token == kInvalidToken; c += kSelThreads) {
+      if (logit_at<kHalf>(logits, base + c) == low) token = static_cast<uint32_t>(c);
+    }
+  }
+  token = wave_min_u32(token);
+  if (tid % kWave == 0u) red_t[tid / kWave] = token;
+  __syncthreads();
+  if (tid == 0) {
+#pragma unroll
+    for (int i = 1; i < kSelWaves; ++i) token = __builtin_elementwise_min(token, red_t[i]);
     // src/cuda/greedy.cu:57: no comparable value selects token 0
-    tokens[blockIdx.x] = best.token == kInvalidToken ? 0u : best.token;
+    tokens[blockIdx.x] = token == kInvalidToken ? 0u : token;
   }
 }
 
@@ -777,10 +892,10 @@ hipError_t launch_linear_f16_simple(const uint16_t* input, const uint16_t* weigh
 hipError_t launch_greedy(const void* logits, bool half, uint32_t* tokens,
                          uint32_t rows, uint32_t vocab, hipStream_t stream) {
   if (half) {
-    hipLaunchKernelGGL((greedy_kernel<true>), dim3(rows), dim3(kThreads), 0, stream,
+    hipLaunchKernelGGL((greedy_kernel<true>), dim3(rows), dim3(kSelThreads), 0, stream,
                        logits, tokens, vocab);
   } else {
-    hipLaunchKernelGGL((greedy_kernel<false>), dim3(rows), dim3(kThreads), 0, stream,
+    hipLaunchKernelGGL((greedy_kernel<false>), dim3(rows), dim3(kSelThreads), 0, stream,
                        logits, tokens, vocab);
   }
   return hipGetLastError();

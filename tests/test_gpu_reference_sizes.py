@@ -1,0 +1,55 @@
+"""The reference operators at the sizes where their kernels change path:
+words and scalars of a row, segments and lanes of a norm, tiles of a
+projection.  Selections and norms are exact; the projection's tolerance is
+derived from its sums."""
+import numpy as np
+import pytest
+
+import oracle
+from tests.gpu_util import B, dev, empty, host, ok, stream
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _lib(hip):
+    return hip
+
+
+@pytest.mark.parametrize("half", [True, False])
+@pytest.mark.parametrize("rows,vocab", [
+    (1, 1), (2, 3), (5, 7), (3, 9), (3, 8191), (2, 8192), (4, 8193), (3, 65535), (2, 131075)])
+def test_greedy_words_scalars_and_special_values(rows, vocab, half):
+    """Rows that start at every offset in a word (odd vocabularies), one word,
+    one batch of words and more, with ties, NaN (quiet and signalling),
+    infinities and signed zeros at the edges."""
+    from market_sim_amd import ops
+    rng = np.random.default_rng(vocab + rows)
+    for special in range(6):
+        x = rng.standard_normal((rows, vocab)).astype(np.float32)
+        x = np.round(x * 8) / 8          # many exact ties, also at the maximum
+        if special == 1:
+            x[:] = -np.inf               # no value above -inf: the lowest id
+            x[:, : vocab // 3] = np.nan
+        elif special == 2:
+            x[:] = np.nan                # nothing comparable: token 0
+        elif special == 3:
+            x = -np.abs(x)
+            x[:, vocab // 2:] = -0.0     # -0 and +0 tie
+            x[:, vocab - 1] = 0.0
+        elif special == 4:
+            x[:, vocab - 1] = np.inf     # the last scalar
+        elif special == 5:
+            x[:, 0] = 100.0              # the first, among NaN
+            x[:, 1::2] = np.nan
+        bits = x.astype(np.float16).view(np.uint16) if half else x.view(np.uint32)
+        if special == 5:                 # signalling NaN: the quiet bit off
+            bits = np.where(np.isnan(x), 0x7C01 if half else 0x7F800001, bits).astype(bits.dtype)
+        out = empty(rows, np.uint32)
+        ld = dev(bits)
+        op = ops.greedy_select_f16 if half else ops.greedy_select_f32
+        ok(op(B(ld), B(out), rows, vocab, stream()))
+        v = np.where(np.isnan(x), -np.inf, x)
+        best = v.max(1, keepdims=True)
+        want = np.argmax((v == best) & ~np.isnan(x), axis=1)   # 0 where all are NaN
+        assert host(out, np.uint32).tolist() == want.tolist(), special
