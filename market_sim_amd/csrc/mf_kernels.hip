@@ -130,6 +130,140 @@ __global__ __launch_bounds__(kWave) void rms_norm_kernel(
   }
 }
 
+// The same norm for many rows: a wave takes 64 / G rows, G lanes a row
+// (split by norm_split).  Lane k of a row holds segment k of it, S
+// 16-byte words, in registers; the running sums go through the segments in
+// order, handed one lane up (DPP) after each, so every row of the wave is in
+// its chain at once and the additions and their order are the reference's.
+// An FP16 square is exact in FP32, so fma(x, x, s) is the reference's rounded
+// square and sum in one instruction on the packed halves.
+// The rows are read once, in contiguous words that stay in registers for the
+// output; the segments are dealt through LDS (a lane's segment at an odd
+// number of 16-byte words, so 16 lanes meet 16 bank groups).
+// Bound: with a wave a SIMD or fewer the chain (H dependent additions, about
+// 5 cycles each), beyond that the SIMDs' issue of H additions per wave.
+// 2048 x 2048 FP16: 25.3 -> 9.4 us a call, FP32 28.5 -> 12.8; 8192 x 4096
+// FP16: 300 -> 45 us, FP32 282 -> 73 (3.7 TB/s); 1 x 576: 5.7 -> 5.6 (from one
+// row a wave with x, its squares and the weight in LDS, which held six rows of
+// 2048 a compute unit; that kernel keeps the rows that are not whole words, or
+// wider).
+struct NormSplit {
+  uint32_t lanes_log2;  // G
+  uint32_t per_wave;    // rows per wave, at most 64 / G
+  uint32_t words;       // 16-byte words per row
+  uint32_t row_magic;   // q / words = q * row_magic >> 20 for q < 1024
+};
+constexpr uint32_t kNormSegMax = 16;   // words per segment: 4, 8, 12 or 16
+constexpr uint32_t kNormWaves = 1024;  // waves (one a SIMD) before waves take more rows
+
+template <bool kHalf, uint32_t kSeg>
+__global__ __launch_bounds__(kWave) void rms_norm_rows_kernel(const void* input,
+                                                              const void* __restrict__ weight,
+                                                              void* output, uint32_t rows,
+                                                              uint32_t H, float epsilon,
+                                                              NormSplit d) {
+  constexpr uint32_t kStride = kSeg | 1u;
+  __shared__ uint4 seg_lds[kWave * kStride];
+  const uint32_t lane = threadIdx.x;
+  const uint32_t first = blockIdx.x * d.per_wave;
+  const uint32_t n = (rows - first < d.per_wave ? rows - first : d.per_wave) * d.words;
+  const uint4* src = static_cast<const uint4*>(input) + static_cast<uint64_t>(first) * d.words;
+  uint4* dst = static_cast<uint4*>(output) + static_cast<uint64_t>(first) * d.words;
+  const uint4* wsrc = static_cast<const uint4*>(weight);
+  // word lane + 64 i of the wave's rows (past the end: the last word again,
+  // read, dealt and written with the same value), at most kSeg per lane
+  uint32_t at = lane;
+  auto word_at = [&](uint32_t i) {
+    const uint32_t q = at + kWave * i;
+    return q < n ? q : n - 1u;
+  };
+  uint4 v[kSeg];
+#pragma unroll
+  for (uint32_t i = 0; i < kSeg; ++i) v[i] = src[word_at(i)];
+#pragma unroll
+  for (uint32_t i = 0; i < kSeg; ++i) {
+    const uint32_t q = word_at(i);
+    const uint32_t j = (q * d.row_magic) >> 20;
+    const uint32_t w = q - j * d.words;
+    const uint32_t k = w / kSeg;
+    seg_lds[((j << d.lanes_log2) + k) * kStride + (w - k * kSeg)] = v[i];
+  }
+  wave_sync();
+  const uint32_t begin = (lane & ((1u << d.lanes_log2) - 1u)) * kSeg;
+  const uint32_t have = begin < d.words ? d.words - begin : 0u;
+  uint4 sg[kSeg];
+#pragma unroll
+  for (uint32_t p = 0; p < kSeg; ++p) sg[p] = seg_lds[lane * kStride + p];
+#pragma unroll
+  for (uint32_t p = 0; p < kSeg; ++p) {
+    const uint32_t keep = p < have ? ~0u : 0u;  // past the row: zeros, which add nothing
+    sg[p] = uint4{sg[p].x & keep, sg[p].y & keep, sg[p].z & keep, sg[p].w & keep};
+    if constexpr (!kHalf) {
+      const float f[4] = {as_float(sg[p].x), as_float(sg[p].y), as_float(sg[p].z), as_float(sg[p].w)};
+      sg[p] = uint4{as_u32(f[0] * f[0]), as_u32(f[1] * f[1]), as_u32(f[2] * f[2]), as_u32(f[3] * f[3])};
+    }
+  }
+  const uint32_t segments = (d.words + kSeg - 1u) / kSeg;
+  // Every lane adds its segment to what it was handed; the lane that holds
+  // segment t after t hand-overs holds the row's sum so far.
+  float s = 0.0f;
+  for (uint32_t t = 0; t < segments; ++t) {
+    if (t != 0u) s = lane_shift_right(s);
+#pragma unroll
+    for (uint32_t p = 0; p < kSeg; ++p) {
+      const uint32_t q[4] = {sg[p].x, sg[p].y, sg[p].z, sg[p].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (kHalf) {
+          const half2_t h = __builtin_bit_cast(half2_t, q[e]);
+          s = __builtin_fmaf(static_cast<float>(h.x), static_cast<float>(h.x), s);
+          s = __builtin_fmaf(static_cast<float>(h.y), static_cast<float>(h.y), s);
+        } else {
+          s = s + as_float(q[e]);
+        }
+      }
+    }
+  }
+  const float inverse = norm_inverse(s, H, epsilon);  // the row's in lane `segments` - 1 of it
+  // the words' places are worked out again: kept over the chain they would
+  // cost a register each
+  asm volatile("" : "+v"(at));
+  constexpr uint32_t kBatch = 4;
+#pragma unroll
+  for (uint32_t i0 = 0; i0 < kSeg; i0 += kBatch) {
+    if (kWave * i0 >= n) break;
+    uint4 g[kBatch];
+    float inv[kBatch];
+#pragma unroll
+    for (uint32_t u = 0; u < kBatch; ++u) {
+      const uint32_t q = word_at(i0 + u);
+      const uint32_t j = (q * d.row_magic) >> 20;
+      g[u] = wsrc[q - j * d.words];
+      inv[u] = __shfl(inverse, static_cast<int>((j << d.lanes_log2) + segments - 1u));
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < kBatch; ++u) {
+      const uint32_t x[4] = {v[i0 + u].x, v[i0 + u].y, v[i0 + u].z, v[i0 + u].w};
+      const uint32_t w[4] = {g[u].x, g[u].y, g[u].z, g[u].w};
+      uint32_t y[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (kHalf) {
+          const half2_t a = __builtin_bit_cast(half2_t, x[e]);
+          const half2_t b = __builtin_bit_cast(half2_t, w[e]);
+          const float y0 = (static_cast<float>(a.x) * inv[u]) * static_cast<float>(b.x);
+          const float y1 = (static_cast<float>(a.y) * inv[u]) * static_cast<float>(b.y);
+          y[e] = static_cast<uint32_t>(float_to_half_rne(y0)) |
+                 (static_cast<uint32_t>(float_to_half_rne(y1)) << 16);
+        } else {
+          y[e] = as_u32((as_float(x[e]) * inv[u]) * as_float(w[e]));
+        }
+      }
+      dst[word_at(i0 + u)] = uint4{y[0], y[1], y[2], y[3]};
+    }
+  }
+}
+
 // Rows too wide to stage whole in LDS (H > kNormStagedMax): the squares are
 // staged kNormChunk features at a time and lane 0 adds them in feature order
 // (one running sum across the chunks: the same chain as the staged kernel),
@@ -834,11 +968,64 @@ hipError_t launch_read_floor(const void* address, uint64_t bytes, uint32_t* sink
   return hipGetLastError();
 }
 
+// The split of rms_norm_rows_kernel, if the call is one for it: whole
+// aligned 16-byte words per row, at most 64 segments of kNormSegMax words.
+// As few lanes per row as hold it (fewer hand-overs, more rows per wave).
+static bool norm_split(const void* input, const void* weight, const void* output, bool half,
+                       uint32_t rows, uint32_t hidden, NormSplit& d, uint32_t& seg) {
+  const uint32_t per = half ? 8u : 4u;
+  if (hidden % per != 0 || hidden / per > kNormSegMax * kWave ||
+      ((reinterpret_cast<uintptr_t>(input) | reinterpret_cast<uintptr_t>(weight) |
+        reinterpret_cast<uintptr_t>(output)) & 15u) != 0) {
+    return false;
+  }
+  d.words = hidden / per;
+  d.lanes_log2 = 0;
+  while (d.words > kNormSegMax << d.lanes_log2) ++d.lanes_log2;
+  seg = (((d.words + (1u << d.lanes_log2) - 1u) >> d.lanes_log2) + 3u) & ~3u;
+  d.per_wave = 1;
+  while (rows / (2u * d.per_wave) >= kNormWaves && 2u * d.per_wave <= 64u >> d.lanes_log2) {
+    d.per_wave *= 2u;
+  }
+  d.row_magic = ((1u << 20) + d.words - 1u) / d.words;
+  return true;
+}
+
+template <bool kHalf>
+static void launch_norm_rows(const void* input, const void* weight, void* output, uint32_t rows,
+                             uint32_t hidden, float epsilon, const NormSplit& d, uint32_t seg,
+                             hipStream_t stream) {
+  const dim3 grid((rows + d.per_wave - 1u) / d.per_wave), block(kWave);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, stream, input, weight, output, rows, hidden, epsilon, d);
+  };
+  if (seg == 4u) {
+    go(rms_norm_rows_kernel<kHalf, 4>);
+  } else if (seg == 8u) {
+    go(rms_norm_rows_kernel<kHalf, 8>);
+  } else if (seg == 12u) {
+    go(rms_norm_rows_kernel<kHalf, 12>);
+  } else {
+    go(rms_norm_rows_kernel<kHalf, 16>);
+  }
+}
+
 hipError_t launch_rms_norm(const void* input, bool half_input, const void* weight,
                            bool half_weight, void* output, bool half_output,
                            float* row_norm, uint32_t rows, uint32_t hidden,
                            float epsilon, hipStream_t stream) {
   const dim3 grid(rows), block(kWave);
+  NormSplit split{};
+  uint32_t seg = 0;
+  if (half_input == half_weight && half_input == half_output && row_norm == nullptr &&
+      norm_split(input, weight, output, half_input, rows, hidden, split, seg)) {
+    if (half_input) {
+      launch_norm_rows<true>(input, weight, output, rows, hidden, epsilon, split, seg, stream);
+    } else {
+      launch_norm_rows<false>(input, weight, output, rows, hidden, epsilon, split, seg, stream);
+    }
+    return hipGetLastError();
+  }
   if (hidden > kNormStagedMax) {
     if (row_norm != nullptr && hidden > 65536u) return hipErrorInvalidValue;  // bound's margin
     if (half_input && half_weight && half_output) {

@@ -53,3 +53,32 @@ def test_greedy_words_scalars_and_special_values(rows, vocab, half):
         best = v.max(1, keepdims=True)
         want = np.argmax((v == best) & ~np.isnan(x), axis=1)   # 0 where all are NaN
         assert host(out, np.uint32).tolist() == want.tolist(), special
+
+
+@pytest.mark.parametrize("rows,hidden", [
+    (1, 4), (1, 8), (3, 520), (1023, 576), (1025, 72), (2048, 1000), (2049, 2048), (4099, 960),
+    (8195, 520), (2050, 4096), (5, 8192), (3, 8200), (4, 4100)])
+def test_rms_norm_segments_bit_exact(rows, hidden):
+    """One row a wave to eight, full and partial segments and last waves, the
+    widest row of the registers and the first past it, in place."""
+    from market_sim_amd import ops
+    rng = np.random.default_rng(rows + hidden)
+    x = (rng.standard_normal((rows, hidden)) * 3).astype(np.float32)
+    w = (1 + 0.02 * rng.standard_normal(hidden)).astype(np.float32)
+    x[0, :] *= 1e-6                       # FP16 subnormals
+    x16, w16 = x.astype(np.float16).view(np.uint16), w.astype(np.float16).view(np.uint16)
+    xd, wd = dev(x), dev(w)
+    ok(ops.rms_norm_f32(B(xd), B(wd), B(xd), rows, hidden, 1e-5, stream()))
+    got = host(xd, np.float32).reshape(rows, hidden)
+    assert np.array_equal(got.view(np.uint32), oracle.rms_norm_f32(x, w, 1e-5).view(np.uint32))
+    xd, wd = dev(x16), dev(w16)
+    out = empty(rows * hidden, np.uint16)
+    ok(ops.rms_norm_f16(B(xd), B(wd), B(out), rows, hidden, 1e-5, stream()))
+    # (x * inverse) * weight leaves the FP32 multiplier as a half, rounded once
+    # from the exact product (v_fma_mixlo_f16): x * inverse comes from the FP32
+    # norm under a weight of one, and its product with a half fits a float64
+    scaled = oracle.rms_norm_f32(x16.view(np.float16).astype(np.float32),
+                                 np.ones(hidden, np.float32), 1e-5)
+    # (its zero addend makes a negative zero positive)
+    want = (scaled.astype(np.float64) * w16.view(np.float16).astype(np.float64) + 0.0).astype(np.float16)
+    assert np.array_equal(host(out, np.uint16).reshape(rows, hidden), want.view(np.uint16))
