@@ -441,6 +441,9 @@ mf_status mf_linear_f16(mf_buffer input, mf_buffer weight, mf_buffer output, uin
     p.H = static_cast<uint32_t>(input_features);
     p.V = static_cast<uint32_t>(output_features);
     p.out_f16 = ptr<uint16_t>(output.address);
+    if (rows <= mf::kStreamRowsMax) {
+      return launch_status(mf::launch_stream_linear(p, device_cus(), native(stream)));
+    }
     return launch_status(mf::launch_projection(p, native(stream)));
   }
   return launch_status(mf::launch_linear_f16_simple(
@@ -455,12 +458,14 @@ mf_status mf_linear_f16(mf_buffer input, mf_buffer weight, mf_buffer output, uin
 namespace {
 
 constexpr uint32_t kFullTile = 256;  // selection over projected scores
+constexpr uint64_t kScratchBytes = 16ull << 20;  // the array of mf_decode_tail_f16_noalloc
 
 struct TailLayout {
   uint64_t y, row_inv, row_norm, row_slack, row_meta, y_hi, y_lo, fb_map, records, fb_records,
       fb_panel, fb_slot_row, fb_slot_norm, fb_slot_slack, scores, tok_norm, range_index,
       row_tiles, dense_spans, dense_flag, total;
   uint32_t tile, max_tiles, fb_tiles, fb_rows;
+  uint32_t fb_blocks;  // the stream head's 16-token blocks per tile
   uint64_t short_counts, short_records;
   uint32_t short_per_part, short_parts;
   bool pass;   // the table pass serves both kinds of rows
@@ -650,11 +655,12 @@ mf_status validate_tail(const mf_decode_tail_args* a, bool full, TailLayout& L) 
     L.tile = gather_tile(a->hidden, a->rows, a->max_count);
     L.max_tiles = static_cast<uint32_t>(a->max_count == 0 ? 1 : (a->max_count + L.tile - 1) / L.tile);
   }
-  L.fb_tiles = mf::fallback_tiles(static_cast<uint32_t>(a->vocab));
   // table pass: one record per (row, 192-token range) holding its ids
   L.pass = !full && table_pass(a);
   L.fused = !full && !L.pass && short_plan(a, L.short_per_part, L.short_parts);
   L.dense = !full && !L.pass && !L.fused && dense_head(a);
+  const uint32_t vocab = static_cast<uint32_t>(a->vocab);
+  L.fb_tiles = mf::fallback_tiles(vocab);
   if (L.pass) {
     const uint64_t longest = a->max_count == 0 ? 1 : a->max_count;
     L.max_tiles = static_cast<uint32_t>(longest < L.fb_tiles ? longest : L.fb_tiles);
@@ -666,42 +672,56 @@ mf_status validate_tail(const mf_decode_tail_args* a, bool full, TailLayout& L) 
   // the dense head's slots: the unrestricted rows, then any row
   const uint64_t fb_slots = L.dense ? fb_rows + rows : fb_rows;
   const uint64_t panel_rows = L.dense ? 0u : fb_rows;
-  uint64_t off = 0;
-  auto take = [&off](uint64_t bytes) {
-    const uint64_t at = off;
-    off = align256(off + bytes);
-    return at;
+  auto place = [&]() {
+    uint64_t off = 0;
+    auto take = [&off](uint64_t bytes) {
+      const uint64_t at = off;
+      off = align256(off + bytes);
+      return at;
+    };
+    // the one-kernel tail's arrival counters: at the start of every layout,
+    // which no other path writes, so they stay zero between calls whatever
+    // the calls' shapes
+    L.short_counts = take(mf::kShortCountRows * 4u);
+    L.short_records = take(L.fused && L.short_parts > 1u
+                               ? rows * L.short_parts * sizeof(mf::ShortPartRecord)
+                               : 0u);
+    L.y = take(xe * 4u);
+    L.row_inv = take(rows * 4u);
+    L.row_norm = take(rows * 4u);
+    L.row_slack = take(rows * 4u);
+    L.row_meta = take(rows * sizeof(mf::RowMeta));
+    const bool split = full || mfma_gather(a->hidden);
+    L.y_hi = take(split ? xe * 2u : 0u);
+    L.y_lo = take(split ? xe * 2u : 0u);
+    L.fb_map = take(rows * 4u);
+    L.records = take(rows * L.max_tiles * sizeof(mf::TileRecord));
+    L.fb_records = take(fb_slots * L.fb_tiles * sizeof(mf::TileRecord));
+    L.fb_panel = take(mf::panel_tiles(static_cast<uint32_t>(panel_rows)) *
+                      mf::panel_tile_bytes(a->hidden));
+    L.fb_slot_row = take(panel_rows * 4u);
+    L.fb_slot_norm = take(panel_rows * 4u);
+    L.fb_slot_slack = take(panel_rows * 4u);
+    L.scores = take(full ? rows * a->vocab * 4u : 0u);
+    L.tok_norm = take(full ? a->vocab * 4u : 0u);
+    L.range_index = take(L.pass ? L.fb_tiles * rows * 16u : 0u);
+    L.row_tiles = take(L.pass ? rows * 4u : 0u);
+    L.dense_spans = take(L.dense ? static_cast<uint64_t>(L.fb_tiles) * rows * 32u : 0u);
+    L.dense_flag = take(L.dense ? rows * 4u : 0u);
+    L.total = off;
   };
-  // the one-kernel tail's arrival counters: at the start of every layout,
-  // which no other path writes, so they stay zero between calls whatever
-  // the calls' shapes
-  L.short_counts = take(mf::kShortCountRows * 4u);
-  L.short_records = take(L.fused && L.short_parts > 1u
-                             ? rows * L.short_parts * sizeof(mf::ShortPartRecord)
-                             : 0u);
-  L.y = take(xe * 4u);
-  L.row_inv = take(rows * 4u);
-  L.row_norm = take(rows * 4u);
-  L.row_slack = take(rows * 4u);
-  L.row_meta = take(rows * sizeof(mf::RowMeta));
-  const bool split = full || mfma_gather(a->hidden);
-  L.y_hi = take(split ? xe * 2u : 0u);
-  L.y_lo = take(split ? xe * 2u : 0u);
-  L.fb_map = take(rows * 4u);
-  L.records = take(rows * L.max_tiles * sizeof(mf::TileRecord));
-  L.fb_records = take(fb_slots * L.fb_tiles * sizeof(mf::TileRecord));
-  L.fb_panel = take(mf::panel_tiles(static_cast<uint32_t>(panel_rows)) *
-                    mf::panel_tile_bytes(a->hidden));
-  L.fb_slot_row = take(panel_rows * 4u);
-  L.fb_slot_norm = take(panel_rows * 4u);
-  L.fb_slot_slack = take(panel_rows * 4u);
-  L.scores = take(full ? rows * a->vocab * 4u : 0u);
-  L.tok_norm = take(full ? a->vocab * 4u : 0u);
-  L.range_index = take(L.pass ? L.fb_tiles * rows * 16u : 0u);
-  L.row_tiles = take(L.pass ? rows * 4u : 0u);
-  L.dense_spans = take(L.dense ? static_cast<uint64_t>(L.fb_tiles) * rows * 32u : 0u);
-  L.dense_flag = take(L.dense ? rows * 4u : 0u);
-  L.total = off;
+  place();
+  if (!L.pass && !L.dense && fb_rows > 0) {
+    // the stream head's tiles: as fine as its compute units want, or coarse
+    // when only that keeps the workspace within the no-allocation array
+    for (const bool coarse : {true, false}) {
+      const TailLayout before = L;
+      L.fb_blocks = mf::stream_tile_blocks(vocab, coarse);
+      L.fb_tiles = mf::stream_tiles(vocab, L.fb_blocks);
+      place();
+      if (!coarse && before.total <= kScratchBytes && L.total > kScratchBytes) L = before;
+    }
+  }
   return ok();
 }
 
@@ -961,7 +981,7 @@ mf_status decode_tail_stage(const mf_decode_tail_args* args, uintptr_t stream, S
         break;
       }
       if (a->unrestricted_count == 0 || L.pass || L.fused) break;
-      e = mf::launch_fallback(fallback_args(a, L, ws), s);
+      e = mf::launch_stream_head(fallback_args(a, L, ws), L.fb_blocks, s);
       break;
     }
     case Stage::kFinalize:
@@ -1058,7 +1078,6 @@ namespace {
 // module load to process end.  Host code never passes the array's name to a
 // kernel or a copy (on the host it is a stand-in, not a device address): it
 // takes the device address from hipGetSymbolAddress, once per device.
-constexpr uint64_t kScratchBytes = 16ull << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 struct ScratchSlot {

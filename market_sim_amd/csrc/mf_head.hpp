@@ -1,7 +1,6 @@
-// The MFMA head's tile pieces shared by the head kernels (mf_mfma.hip) and
-// the table pass (mf_pass.hip): slot metadata of a panel tile, the per-tile
-// accumulators and the windowed-argmax epilogue that turns a tile's scores
-// into window records.
+// Pieces of the heads' windowed-argmax epilogue: a panel tile's slot
+// metadata, and the table pass's (mf_pass.hip) per-tile accumulators and
+// window records.  The stream head (mf_stream.hip) shares the lane layout.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -14,41 +13,24 @@ namespace {
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 
-// ---- MFMA head of the unrestricted rows -----------------------------------
+// ---- unrestricted rows in the table pass -----------------------------------
 //
-// A workgroup owns the 32 slots of one panel tile (an M-tile) and a run of
-// 192-token tiles (one window record per row and tile); the runs are sized
-// so that every compute unit gets the same number of tiles.  The tile's 12
-// blocks of 16 tokens are split over the waves, kBlocks per wave; each block
-// is one v_mfma_f32_16x16x32_f16 column block against the 32 slots as four
-// 16-row A blocks: A rows 2j and 2j + 1 of block rb are the hi and lo halves
-// of slot 8 rb + j.  In the 16x16x32 layout lane l holds 8 consecutive
-// features of column / A row l % 16 at k-block l / 16, so the four lanes of
-// a token read 64 contiguous bytes per step, and table rows go straight from
-// memory into the MFMA registers.  A second MFMA of each token block with
-// itself gives the squared token norms (Gram diagonal) for the error bound.
-//
-// Two variants:
-//   narrow rows (panel tile in LDS, H <= 576): at entry the workgroup copies
-//     its panel tile into LDS with 1 KiB global-to-LDS bursts and every wave
-//     issues the loads of its whole K range; one wait, one barrier, then the
-//     MFMAs.  Each tile costs one memory round trip.
-//   wide rows: A and B from memory (A from L2) in units of KC steps, two
-//     units in flight.
+// A workgroup scores the 32 slots of a panel tile against its 192-token tile
+// (one window record per row and tile).  The tile's 12 blocks of 16 tokens
+// are split over the waves, kBlocks per wave; each block is one
+// v_mfma_f32_16x16x32_f16 column block against the slots' FP16 hi as two
+// 16-row A blocks: A row j of block rb is slot 16 rb + j.  In the 16x16x32
+// layout lane l holds 8 consecutive features of column / A row l % 16 at
+// k-block l / 16.  A second MFMA of each token block with itself gives the
+// squared token norms (Gram diagonal) for the error bound.
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 constexpr uint32_t kHeadTileBlocks = kHeadTileTokens / 16;
-// narrow-row variant: waves per workgroup (tile blocks per wave = 12 / waves)
-constexpr int kHeadLdsWaves = 4;
-// wide-row variant: 4 waves x 3 blocks
-constexpr int kWideWaves = 4;
-constexpr int kWideBlocks = 3;
-
 // The tile's scores [slot][token] and token norm bounds, staged in LDS for
 // the epilogue (rows padded so the four slot rows one write instruction
 // touches fall on different banks).
 constexpr uint32_t kEpiStride = kHeadTileTokens + 8;
-constexpr int kEpiWaves = 4;  // both variants run four waves
+constexpr int kEpiWaves = 4;
 struct HeadEpi {
   float g[kPanelRows][kEpiStride];
   float tn[kEpiWaves];             // per-wave token-norm maxima
@@ -57,7 +39,7 @@ struct HeadEpi {
 
 template <int kBlocks>
 struct HeadAcc {
-  floatx4 acc[4][kBlocks];
+  floatx4 acc[2][kBlocks];
   floatx4 gram[kBlocks];
 };
 
@@ -129,11 +111,9 @@ __device__ __forceinline__ float lane8_max(float v) {
 }
 
 // The tile's window records.  Lane l holds D[4 (l / 16) + i][l % 16] of
-// each block: A rows 2j, 2j + 1 (hi, lo of slot 8 rb + j) for j = 2 kb and
-// 2 kb + 1, so the score of slot 8 rb + 2 kb + jj (jj = 0, 1) and token
-// (wave kBlocks + tb) 16 + col of the tile is acc[rb][tb][2 jj] +
-// acc[rb][tb][2 jj + 1]; the Gram diagonal of column c sits in lane
-// c + 16 (c / 4), element c % 4.
+// each block, so the score of slot 16 rb + 4 kb + i and token
+// (wave kBlocks + tb) 16 + col of the tile is acc[rb][tb][i]; the Gram
+// diagonal of column c sits in lane c + 16 (c / 4), element c % 4.
 //
 // One bound per slot and tile: b = tn_max (coef ||z|| + coef2) + slack with
 // tn_max the largest token-norm bound of the tile, which is at least every
@@ -143,11 +123,7 @@ __device__ __forceinline__ float lane8_max(float v) {
 // 8 w + s, 24 consecutive tokens each, so the eight slots of a wave share
 // every instruction; members come out in ascending token order.  Ends with
 // a barrier (LDS is reused by the next tile).
-//
-// kHiOnly: A rows are the slots' FP16 hi alone, A row j of block rb being
-// slot 16 rb + j (blocks rb = 0, 1), so the score of slot 16 rb + 4 kb + i
-// is acc[rb][tb][i].
-template <int kWaves, int kBlocks, bool kHiOnly = false>
+template <int kWaves, int kBlocks>
 __device__ __forceinline__ void head_records(const FallbackArgs& f, const HeadAcc<kBlocks>& h,
                                              HeadEpi& epi, const uint32_t* src_row,
                                              const float* src_norm, const float* src_slack,
@@ -170,20 +146,10 @@ __device__ __forceinline__ void head_records(const FallbackArgs& f, const HeadAc
                             : (e == 1u ? h.gram[tb][1] : (e == 2u ? h.gram[tb][2] : h.gram[tb][3]));
     // lanes of the Gram diagonal, tokens of the vocabulary
     if (col / 4u == kb && t < nt) tn_local = __builtin_fmaxf(tn_local, __fsqrt_rn(d) * (1.0f + 0x1p-7f));
-    if constexpr (kHiOnly) {
 #pragma unroll
-      for (int rb = 0; rb < 2; ++rb) {
+    for (int rb = 0; rb < 2; ++rb) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) epi.g[rb * 16 + 4 * kb + i][t] = h.acc[rb][tb][i];
-      }
-    } else {
-#pragma unroll
-      for (int rb = 0; rb < 4; ++rb) {
-#pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
-          epi.g[rb * 8 + 2 * kb + jj][t] = h.acc[rb][tb][2 * jj] + h.acc[rb][tb][2 * jj + 1];
-        }
-      }
+      for (int i = 0; i < 4; ++i) epi.g[rb * 16 + 4 * kb + i][t] = h.acc[rb][tb][i];
     }
   }
   // a NaN norm (a non-finite table row) propagates: the bound then fails the

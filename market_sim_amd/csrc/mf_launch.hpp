@@ -299,16 +299,28 @@ struct FallbackArgs {
   const uint16_t* emb;
   uint32_t H;
   uint32_t V;
-  TileRecord* records;      // [m, tiles] (fallback_tiles(V) tiles of 192 tokens)
+  TileRecord* records;      // [m, tiles] (table pass: 192-token tiles)
   uint32_t* fb_map;         // [rows] written: row -> slot
-  uint32_t groups;          // compute units: workgroups per M-tile
-  uint32_t tiles_per_group; // set by the launcher
+  uint32_t groups;          // compute units
+  uint32_t tiles_per_group; // table pass: set by its launcher
   float coef;               // b = ||e|| * (coef * ||z|| + coef2) + slot slack
   float coef2;
 };
 
-uint32_t fallback_tiles(uint32_t vocab);
-hipError_t launch_fallback(const FallbackArgs& args, hipStream_t stream);
+// 192-token tiles of the table pass and of the dense head
+__host__ __device__ constexpr uint32_t fallback_tiles(uint32_t vocab) {
+  return (vocab + kHeadTileTokens - 1) / kHeadTileTokens;
+}
+
+// ---- few rows against the whole table (mf_stream.hip) -----------------------
+
+constexpr uint32_t kStreamCUs = 256;      // compute units the tiles are cut for
+constexpr uint32_t kStreamRowsMax = 128;  // linear_f16 rows
+// Tiles of 16 `blocks` tokens; blocks of a vocabulary and the tiles they make.
+uint32_t stream_tile_blocks(uint32_t vocab, bool coarse);
+uint32_t stream_tiles(uint32_t vocab, uint32_t blocks);
+hipError_t launch_stream_head(const FallbackArgs& args, uint32_t blocks, hipStream_t stream);
+hipError_t launch_stream_linear(const ProjArgs& args, uint32_t groups, hipStream_t stream);
 
 // ---- table pass (mf_pass.hip) ------------------------------------------------
 //

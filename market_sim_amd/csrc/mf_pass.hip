@@ -262,7 +262,6 @@ __global__ __launch_bounds__(kThreads) void pass_kernel(PassArgs p) {
   constexpr uint32_t H = 32u * kSteps;
   constexpr uint32_t kSlot = slot_bytes(H);
   constexpr uint32_t kTileHalves = static_cast<uint32_t>(panel_tile_bytes(H) / 2u);
-  constexpr uint32_t kPanelSlotHalves = 2u * (H + kPanelPad);  // one panel slot's [hi | lo]
   extern __shared__ __align__(16) unsigned char dyn[];
   __shared__ uint32_t src_row[kPanelRows];
   __shared__ float src_norm[kPanelRows];
@@ -769,8 +768,8 @@ __global__ __launch_bounds__(kThreads) void pass_kernel(PassArgs p) {
       MF_STAMP(13);
       head_lds(h);
       MF_STAMP(14);
-      head_records<kWaves, kBlocks, true>(f, h, epi, src_row, src_norm, src_slack,
-                                          pt * kPanelRows, tile, tiles);
+      head_records<kWaves, kBlocks>(f, h, epi, src_row, src_norm, src_slack,
+                                    pt * kPanelRows, tile, tiles);
     }
   }
   MF_STAMP(15);

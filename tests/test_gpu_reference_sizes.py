@@ -82,3 +82,45 @@ def test_rms_norm_segments_bit_exact(rows, hidden):
     # (its zero addend makes a negative zero positive)
     want = (scaled.astype(np.float64) * w16.view(np.float16).astype(np.float64) + 0.0).astype(np.float16)
     assert np.array_equal(host(out, np.uint16).reshape(rows, hidden), want.view(np.uint16))
+
+
+@pytest.mark.parametrize("rows,inf,outf", [
+    (1, 32, 17), (16, 96, 4129), (17, 64, 5000), (32, 160, 193), (33, 576, 8200), (64, 64, 4097),
+    (65, 1024, 300), (128, 96, 12345), (129, 96, 4097)])
+def test_linear_f16_few_rows_random(rows, inf, outf):
+    """The streamed projection at the edges of its row counts (16, 32, 64,
+    128), with a half chunk of features at the end, partial and single token
+    blocks and an odd output width: every output within half an FP16 ulp plus
+    the FP32 accumulation bound 2 H 2^-24 sum |x w| of the exact product."""
+    from market_sim_amd import ops
+    rng = np.random.default_rng(rows * 7 + inf)
+    x = rng.uniform(-1.0, 1.0, (rows, inf)).astype(np.float16)
+    w = rng.uniform(-1.0, 1.0, (outf, inf)).astype(np.float16)
+    out = empty(rows * outf, np.uint16)
+    xd, wd = dev(x.view(np.uint16)), dev(w.view(np.uint16))
+    ok(ops.linear_f16(B(xd), B(wd), B(out), rows, inf, outf, stream()))
+    got = host(out, np.uint16).reshape(rows, outf).view(np.float16).astype(np.float64)
+    x64, w64 = x.astype(np.float64), w.astype(np.float64)
+    exact = x64 @ w64.T
+    mag = np.abs(x64) @ np.abs(w64).T
+    half_ulp = np.spacing(np.maximum(np.abs(got), np.abs(exact)).astype(np.float16)).astype(
+        np.float64) / 2
+    assert np.all(np.abs(got - exact) <= half_ulp + 2.0 * inf * 2.0 ** -24 * mag)
+
+
+@pytest.mark.parametrize("rows,open_rows,vocab,hidden", [
+    (3, 1, 17, 64), (40, 33, 48, 128), (9, 4, 4097, 576), (70, 65, 8200, 640), (5, 2, 70001, 1088)])
+def test_stream_head_tiles_match_the_oracle(rows, open_rows, vocab, hidden):
+    """Unrestricted rows beside gathered ones: one, two and three panel tiles,
+    tiles of two 16-token blocks up to sixteen, two rounds, a partial last
+    tile, one token past a block."""
+    from market_sim_amd import workloads as wl
+    from market_sim_amd.tail import DeviceTail
+    w = wl.ragged_pack("stream", 3, vocab, hidden, rows, "uniform", max(1, vocab // 20),
+                       open_rows / rows)
+    tok, sc, nx = DeviceTail(w, sorted_lists=False).run()
+    etok, esc, enx = oracle.decode_tail(w.x, w.norm_weight, w.epsilon, w.embedding, w.row_state,
+                                        w.state_offsets, w.state_tokens, threads=8)
+    assert w.unrestricted_rows.size == open_rows
+    assert np.array_equal(tok, etok) and np.array_equal(nx, enx)
+    assert np.array_equal(sc.view(np.uint32), esc.view(np.uint32))
