@@ -444,7 +444,7 @@ mf_status mf_linear_f16(mf_buffer input, mf_buffer weight, mf_buffer output, uin
     if (rows <= mf::kStreamRowsMax) {
       return launch_status(mf::launch_stream_linear(p, device_cus(), native(stream)));
     }
-    return launch_status(mf::launch_projection(p, native(stream)));
+    return launch_status(mf::launch_projection(p, device_cus(), native(stream)));
   }
   return launch_status(mf::launch_linear_f16_simple(
       ptr<const uint16_t>(input.address), ptr<const uint16_t>(weight.address),
@@ -1174,7 +1174,7 @@ mf_status mf_decode_tail_full_f16(const mf_decode_tail_args* args, uintptr_t str
     pj.V = static_cast<uint32_t>(a->vocab);
     pj.out_f32 = scores;
     pj.tok_norm = tok_norm;
-    e = mf::launch_projection(pj, s);
+    e = mf::launch_projection(pj, device_cus(), s);
     if (e != hipSuccess) return launch_status(e);
   }
   // 3. restricted selection over the scores (unrestricted rows: every id),

@@ -285,7 +285,8 @@ struct ProjArgs {
   float* tok_norm;     // [V] ||e_t|| upper bounds, written by M-tile 0 (or null)
 };
 
-hipError_t launch_projection(const ProjArgs& args, hipStream_t stream);
+// groups: compute units (whole XCDs of them are used)
+hipError_t launch_projection(const ProjArgs& args, uint32_t groups, hipStream_t stream);
 
 // Full-vocabulary head for unrestricted rows: projection with a windowed
 // argmax epilogue, per-tile records and a last-arriver merge per row that

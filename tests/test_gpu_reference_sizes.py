@@ -86,11 +86,12 @@ def test_rms_norm_segments_bit_exact(rows, hidden):
 
 @pytest.mark.parametrize("rows,inf,outf", [
     (1, 32, 17), (16, 96, 4129), (17, 64, 5000), (32, 160, 193), (33, 576, 8200), (64, 64, 4097),
-    (65, 1024, 300), (128, 96, 12345), (129, 96, 4097)])
-def test_linear_f16_few_rows_random(rows, inf, outf):
+    (65, 1024, 300), (128, 96, 12345), (129, 96, 4097), (700, 160, 9001), (1100, 64, 20008),
+    (1030, 32, 20008)])
+def test_linear_f16_paths_random(rows, inf, outf):
     """The streamed projection at the edges of its row counts (16, 32, 64,
-    128), with a half chunk of features at the end, partial and single token
-    blocks and an odd output width: every output within half an FP16 ulp plus
+    128) and the tiled one past them, several tiles a workgroup: a half chunk
+    of features at the end, partial and single token blocks, odd widths; every output within half an FP16 ulp plus
     the FP32 accumulation bound 2 H 2^-24 sum |x w| of the exact product."""
     from market_sim_amd import ops
     rng = np.random.default_rng(rows * 7 + inf)
