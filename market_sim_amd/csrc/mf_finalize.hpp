@@ -32,6 +32,9 @@ struct FinalizeLds {
   uint32_t* cand_pos;   // [cand_max]
   uint32_t cand_max;
   FinalizeWords* w;
+  // a row's waves (kWaves of finalize_row): this one, and their results
+  uint32_t wave;
+  Best* wave_results;   // [kWaves]
 };
 
 // Reference-order chain over LDS-resident FP32 y and FP16 row (the same
@@ -95,7 +98,8 @@ __device__ float chain_lds(const float* ys, const uint16_t* row, uint32_t H) {
 // steps and their order are those of the reference chain; only the place of
 // the running sum changes.  Candidate c's score ends in lane nseg c + nseg - 1.
 constexpr uint32_t kChainSeg = 64;
-template <bool kMulAdd>
+// The row's waves take the passes in turn.
+template <bool kMulAdd, uint32_t kWaves>
 __device__ __forceinline__ Best rescore_segmented(const FinalizeArgs& a, const FinalizeLds& L,
                                                   uint32_t n) {
   const uint32_t lane = threadIdx.x % kWave;
@@ -105,7 +109,8 @@ __device__ __forceinline__ Best rescore_segmented(const FinalizeArgs& a, const F
   const uint32_t c = lane / nseg;
   const uint32_t k = lane % nseg;
   Best best = best_identity();
-  for (uint32_t base = 0; base < n; base += per_pass) {
+  const uint32_t first = kWaves > 1u ? L.wave * per_pass : 0u;
+  for (uint32_t base = first; base < n; base += kWaves * per_pass) {
     const uint32_t m = n - base < per_pass ? n - base : per_pass;
     const bool active = c < m;
     const uint32_t j = base + (active ? c : 0u);
@@ -148,7 +153,9 @@ __device__ __forceinline__ Best rescore_segmented(const FinalizeArgs& a, const F
 // Rescores candidates cand_token[0..n) of one row in the reference order:
 // in registers (rescore_segmented) when H is a multiple of kChainSeg of at
 // most kWave segments, else stage_rows rows at a time staged in LDS;
-// returns the wave's best.
+// returns the wave's best.  kWaves > 1 (register rescoring only): the best of
+// this wave's share; the candidates must stand in the same order for all.
+template <uint32_t kWaves>
 __device__ inline Best rescore_candidates(const FinalizeArgs& a, const FinalizeLds& L,
                                           uint32_t n) {
   const uint32_t lane = threadIdx.x % kWave;
@@ -156,7 +163,8 @@ __device__ inline Best rescore_candidates(const FinalizeArgs& a, const FinalizeL
   if (H % kChainSeg == 0u && H <= kChainSeg * kWave &&
       (reinterpret_cast<uintptr_t>(a.emb) & 15u) == 0) {
     wave_sync();
-    return a.order == 1 ? rescore_segmented<true>(a, L, n) : rescore_segmented<false>(a, L, n);
+    return a.order == 1 ? rescore_segmented<true, kWaves>(a, L, n)
+                        : rescore_segmented<false, kWaves>(a, L, n);
   }
   Best best = best_identity();
   for (uint32_t base = 0; base < n; base += L.stage_rows) {
@@ -242,13 +250,29 @@ __device__ __forceinline__ float records_lower(const FinalizeArgs& a, uint32_t r
   return q - __builtin_fabsf(q) * 0x1p-20f - 0x1p-126f;
 }
 
-// Finalizes row r (meta = its metadata) with one wave.  stage_y() puts the
+// The best of the row's waves, in every wave.  All of them call it.
+template <uint32_t kWaves>
+__device__ __forceinline__ Best best_of_waves(const FinalizeLds& L, Best b) {
+  if constexpr (kWaves > 1u) {
+    if (threadIdx.x % kWave == 0u) L.wave_results[L.wave] = b;
+    __syncthreads();
+    b = L.wave_results[0];
+#pragma unroll
+    for (uint32_t w = 1; w < kWaves; ++w) b = best_of(b, L.wave_results[w]);
+    __syncthreads();
+  }
+  return b;
+}
+
+// Finalizes row r (meta = its metadata) with one wave, or with kWaves waves
+// that all follow the row's records (the same loads and decisions, candidate
+// buffers of their own) and share its rescoring.  stage_y() puts the
 // row's normalized hidden vector into L.ys; it is called once the record
 // headers are in flight, before the first rescore, so the caller can keep
 // the vector's loads in flight meanwhile.  Writes token, score and next
 // state of the row; rows that are neither gathered nor served by the MFMA
 // head are left alone (their outputs were preset by the norm kernel).
-template <typename StageY>
+template <uint32_t kWaves, typename StageY>
 __device__ inline void finalize_row(const FinalizeArgs& a, uint32_t r, const RowMeta& meta,
                                     const FinalizeLds& L, StageY&& stage_y) {
   const uint32_t lane = threadIdx.x % kWave;
@@ -326,7 +350,7 @@ __device__ inline void finalize_row(const FinalizeArgs& a, uint32_t r, const Row
   const bool invalid = wave_sum_u32(inv) != 0u;
   if (invalid) {
     // an id outside the vocabulary makes the row invalid (greedy.cu:163-166)
-    if (lane == 0) {
+    if (lane == 0 && (kWaves == 1u || L.wave == 0u)) {
       a.out_token[r] = kInvalidToken;
       if (a.out_score != nullptr) a.out_score[r] = __builtin_nanf("");
       uint32_t* next = next_state_slot(a.out_next, a.row_sequence, a.capacity, r);
@@ -378,11 +402,12 @@ __device__ inline void finalize_row(const FinalizeArgs& a, uint32_t r, const Row
               L.cand_token[lane] = virtual_list ? p : a.tokens[meta.list_begin + p];
               L.cand_pos[lane] = p;
             }
-            best = best_of(best, rescore_candidates(a, L, n));
+            best = best_of(best, rescore_candidates<kWaves>(a, L, n));
           }
         }
       }
     }
+    best = best_of_waves<kWaves>(L, best);
     if (best.token != kInvalidToken) lg = __builtin_fmaxf(lg, records_lower(a, r, best.score));
   }
 
@@ -456,7 +481,8 @@ __device__ inline void finalize_row(const FinalizeArgs& a, uint32_t r, const Row
   }
   wave_sync();
   if (nc <= L.cand_max) {
-    if (nc > 0) best = best_of(best, rescore_candidates(a, L, nc));
+    if (nc > 0) best = best_of(best, rescore_candidates<kWaves>(a, L, nc));
+    best = best_of_waves<kWaves>(L, best);
   } else {
     // flushed sweeps: a sweep of sw tiles adds at most sw kTileMembers =
     // cand_max / 2 candidates, so flushing above half keeps the buffer
@@ -475,7 +501,8 @@ __device__ inline void finalize_row(const FinalizeArgs& a, uint32_t r, const Row
       const uint32_t n = L.w->n_cand;
       // flush when the next sweep could overflow the buffer, and at the end
       if (n > 0 && (n > L.cand_max / 2u || t0 + sw >= ntiles)) {
-        best = best_of(best, rescore_candidates(a, L, n));
+        // (appended by atomics, in any order: every wave rescores all of them)
+        best = best_of(best, rescore_candidates<1>(a, L, n));
         wave_sync();
         if (lane == 0) L.w->n_cand = 0u;
         wave_sync();
@@ -507,7 +534,7 @@ __device__ inline void finalize_row(const FinalizeArgs& a, uint32_t r, const Row
     wave_sync();
     score = a.order == 1 ? chain_lds<true>(L.ys, L.es, H) : chain_lds<false>(L.ys, L.es, H);
   }
-  if (lane == 0) {
+  if (lane == 0 && (kWaves == 1u || L.wave == 0u)) {
     uint32_t next = kInvalidToken;
     if (virtual_list) {
       next = kStateUnrestricted;

@@ -435,8 +435,15 @@ __global__ __launch_bounds__(kThreads) void gather_planned_kernel(GatherArgs a) 
 }
 
 // ---------------------------------------------------------------------------
-// K3: finalize (one wave per row; the per-row work is finalize_row in
-// mf_finalize.hpp)
+// K3: finalize (the per-row work is finalize_row in mf_finalize.hpp): one
+// wave per row, or kWideWaves for rows of kWideHidden features and more.  A
+// rescoring pass is a chain of H dependent steps (4.3 us at H = 2048) for only
+// 64 / (H / 64) candidates, and the row with the most of them (a crowded tile
+// is rescored whole) sets the kernel's time; at H = 576 a pass takes seven
+// candidates and nearly every row needs one.  1024 rows of H = 2048,
+// V = 128256 (three inputs): 65.6 -> 44.4 us on average, 124 -> 73 at most; four
+// waves 48.3 / 56 and eight 80.3 (at about 250 registers two waves a SIMD stay, so
+// two waves per row still hold 1024 rows at once, four hold half of them).
 // ---------------------------------------------------------------------------
 
 constexpr uint32_t kStage = 8;  // embedding rows staged in LDS per rescore pass
@@ -451,16 +458,21 @@ __host__ __device__ inline uint32_t finalize_stage_rows(uint32_t H, const void* 
 }
 constexpr uint32_t kCandMax = 2 * kWave * kTileMembers;
 
-template <uint32_t kYRegs>
-__global__ __launch_bounds__(kWave) void finalize_kernel(FinalizeArgs a) {
+constexpr uint32_t kWideHidden = 1024;
+constexpr uint32_t kWideWaves = 2;
+
+template <uint32_t kYRegs, uint32_t kWaves>
+__global__ __launch_bounds__(kWave* kWaves) void finalize_kernel(FinalizeArgs a) {
   extern __shared__ __align__(16) float lds[];
-  __shared__ uint32_t cand_token[kCandMax];
-  __shared__ uint32_t cand_pos[kCandMax];
-  __shared__ FinalizeWords words;
+  __shared__ uint32_t cand_token[kWaves][kCandMax];
+  __shared__ uint32_t cand_pos[kWaves][kCandMax];
+  __shared__ FinalizeWords words[kWaves];
+  __shared__ Best results[kWaves];
+  const uint32_t wave = kWaves > 1u ? threadIdx.x / kWave : 0u;
   const FinalizeLds L{lds, reinterpret_cast<uint16_t*>(lds + a.H), finalize_stage_rows(a.H, a.emb),
-                      cand_token, cand_pos, kCandMax, &words};
+                      cand_token[wave], cand_pos[wave], kCandMax, &words[wave], wave, results};
   const uint32_t r = blockIdx.x;
-  const uint32_t lane = threadIdx.x;
+  const uint32_t lane = threadIdx.x % kWave;
   const RowMeta meta = a.row_meta[r];
   const float* yrow = a.y + static_cast<uint64_t>(r) * a.H;
   if constexpr (kYRegs > 0) {
@@ -474,7 +486,7 @@ __global__ __launch_bounds__(kWave) void finalize_kernel(FinalizeArgs a) {
       const uint32_t q = lane + u * kWave;
       yv[u] = q < n4 ? reinterpret_cast<const float4*>(yrow)[q] : float4{0.0f, 0.0f, 0.0f, 0.0f};
     }
-    finalize_row(a, r, meta, L, [&]() {
+    finalize_row<kWaves>(a, r, meta, L, [&]() {
 #pragma unroll
       for (uint32_t u = 0; u < kYRegs; ++u) {
         const uint32_t q = lane + u * kWave;
@@ -488,7 +500,7 @@ __global__ __launch_bounds__(kWave) void finalize_kernel(FinalizeArgs a) {
     } else {
       for (uint32_t f = lane; f < a.H; f += kWave) L.ys[f] = yrow[f];
     }
-    finalize_row(a, r, meta, L, []() {});
+    finalize_row<kWaves>(a, r, meta, L, []() {});
   }
 }
 
@@ -556,12 +568,21 @@ hipError_t launch_gather(ScoreSource source, const GatherArgs& a, hipStream_t st
 hipError_t launch_finalize(const FinalizeArgs& a, hipStream_t stream) {
   const size_t lds = static_cast<size_t>(a.H) * sizeof(float) +
                      static_cast<size_t>(finalize_stage_rows(a.H, a.emb)) * a.H * sizeof(uint16_t);
+  const dim3 grid(a.rows);
+  auto go = [&](auto kernel, uint32_t waves) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kWave * waves), lds, stream, a);
+  };
+  // several waves share a row's rescoring only where it runs in registers
+  const bool wide = a.H >= kWideHidden && finalize_stage_rows(a.H, a.emb) == 1u;
   if (a.H % 4u == 0 && a.H <= 4u * kWave * 4u) {
-    hipLaunchKernelGGL(finalize_kernel<4>, dim3(a.rows), dim3(kWave), lds, stream, a);
+    if (wide) go(finalize_kernel<4, kWideWaves>, kWideWaves);
+    else go(finalize_kernel<4, 1>, 1u);
   } else if (a.H % 4u == 0 && a.H <= 4u * kWave * 8u) {
-    hipLaunchKernelGGL(finalize_kernel<8>, dim3(a.rows), dim3(kWave), lds, stream, a);
+    if (wide) go(finalize_kernel<8, kWideWaves>, kWideWaves);
+    else go(finalize_kernel<8, 1>, 1u);
   } else {
-    hipLaunchKernelGGL(finalize_kernel<0>, dim3(a.rows), dim3(kWave), lds, stream, a);
+    if (wide) go(finalize_kernel<0, kWideWaves>, kWideWaves);
+    else go(finalize_kernel<0, 1>, 1u);
   }
   return hipGetLastError();
 }
