@@ -58,6 +58,22 @@ def stream_workspace(nbytes: int, stream, device: str):
     return t, ws
 
 
+def order_after(stream, device: str) -> None:
+    """Work enqueued on ``stream`` from here on runs after the work already on
+    the caller's current stream.  An event pair between two streams costs
+    about 10 us of host time and stalls both queues, so it is left out where
+    there is nothing to wait for: on one and the same stream, and when the
+    caller's stream has finished.  (A stream under graph capture cannot be
+    asked; the pair is then part of the graph.)"""
+    import torch
+    current = torch.cuda.current_stream(device)
+    if current == stream:
+        return
+    if not torch.cuda.is_current_stream_capturing() and current.query():
+        return
+    stream.wait_stream(current)
+
+
 def _table_tensor(table, device: str):
     """An FP16 [V, H] table as a device tensor (uint16 bits or float16)."""
     import torch
@@ -154,6 +170,11 @@ class RestrictedDecoder:
         self._ws_t, ws = stream_workspace(nbytes, self.stream, device)
         for a in self._args:
             a.workspace = ws.c()
+        # every step's output rows and the start states, once: a tensor index
+        # costs about as much as the call itself
+        D = ops.DeviceBuffer.of
+        self._outputs = [(D(self.tokens[k]).c(), D(self.scores[k]).c()) for k in range(max_steps)]
+        self._start_states = self.states[0]
         self.k = 0
 
     def _make_args(self, parity: int) -> abi.DecodeTailArgs:
@@ -172,10 +193,12 @@ class RestrictedDecoder:
     def start(self, states: Optional[Sequence[int]] = None) -> None:
         """Every row at the DFA root, or at the given states (one upload)."""
         import torch
-        init = np.zeros(self.rows, np.uint32) if states is None else \
-            np.asarray(states, dtype=np.uint32)
         with torch.cuda.stream(self.stream):
-            self.states[0].copy_(_device_u32(init, self.device))
+            if states is None:
+                self._start_states.zero_()
+            else:
+                init = np.ascontiguousarray(states, dtype=np.uint32)
+                self._start_states.copy_(torch.from_numpy(init.view(np.int32)))
         self.k = 0
 
     def step(self, hidden) -> None:
@@ -186,15 +209,13 @@ class RestrictedDecoder:
             raise RuntimeError(f"decoder holds {self.max_steps} steps")
         if tuple(hidden.shape) != (self.rows, self.hidden) or not hidden.is_contiguous():
             raise ValueError(f"hidden must be a contiguous [{self.rows}, {self.hidden}] tensor")
-        import torch
         # the step runs after the work that produced ``hidden`` on the
         # caller's stream, and the allocator keeps ``hidden`` for this stream
-        self.stream.wait_stream(torch.cuda.current_stream(self.device))
+        order_after(self.stream, self.device)
         hidden.record_stream(self.stream)
         a = self._args[self.k % 2]
-        a.x = ops.DeviceBuffer.of(hidden).c()
-        a.out_token = ops.DeviceBuffer.of(self.tokens[self.k]).c()
-        a.out_score = ops.DeviceBuffer.of(self.scores[self.k]).c()
+        a.x.address, a.x.bytes = hidden.data_ptr(), hidden.nbytes
+        a.out_token, a.out_score = self._outputs[self.k]
         abi.check("decode_tail", ops.decode_tail_f16(a, self.stream.cuda_stream))
         self.k += 1
 
@@ -406,7 +427,7 @@ class SequencePacker:
             raise ValueError("a sequence appears twice in the batch")
         unr = [r for r, i in enumerate(ids) if i in self._unrestricted_ids]
         key = (tuple(entries), tuple(unr))
-        self.stream.wait_stream(torch.cuda.current_stream(self.device))
+        order_after(self.stream, self.device)
         hidden.record_stream(self.stream)
         with torch.cuda.stream(self.stream):
             if key != self._last_pack:

@@ -131,3 +131,32 @@ def test_run_record_of_a_decode_result_passes_the_contract():
         decode.run_record(res, [[1]], table, seed=3, inference_seconds=0.25,
                           model_load_seconds=0.5, peak_gpu_memory_bytes=1,
                           device_name="x", runtime_version="7.0")
+
+
+@pytest.mark.parametrize("same,capturing,pending,waits", [
+    (True, False, True, False),      # one stream: already in order
+    (False, False, False, False),    # the caller's stream has finished
+    (False, False, True, True),
+    (False, True, False, True),      # a capturing stream cannot be asked
+])
+def test_order_after_waits_only_for_pending_work(monkeypatch, same, capturing, pending, waits):
+    import torch
+    log = []
+
+    class Stream:
+        def __init__(self, name):
+            self.name = name
+
+        def query(self):
+            assert not capturing
+            return not pending
+
+        def wait_stream(self, other):
+            log.append((self.name, other.name))
+
+    mine = Stream("loop")
+    caller = mine if same else Stream("caller")
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: caller)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+    decode.order_after(mine, "cuda")
+    assert log == ([("loop", "caller")] if waits else [])
