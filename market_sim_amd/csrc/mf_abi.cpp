@@ -143,7 +143,7 @@ uint32_t device_cus() {
 
 
 uint32_t head_chunk(uint64_t H, uint64_t max_count) {
-  uint32_t c = H == 576 ? 128u : 64u;
+  uint32_t c = H % 8u == 0 ? 128u : 64u;
   while (c < mf::kHeadChunkMax &&
          (max_count + c - 1) / c > mf::kHeadMaxRecords) {
     c *= 2;

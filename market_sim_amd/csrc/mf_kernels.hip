@@ -364,17 +364,23 @@ __device__ RowList resolve_row(const HeadArgs& a, uint32_t r) {
   return l;
 }
 
-// Cross-wave reduction scratch of a 256-thread block.
+// Cross-wave reduction scratch of a workgroup of kW waves.
+template <int kW>
 struct Red {
-  float red_f[kWaves];
-  uint32_t red_u[kWaves];
-  uint32_t red_u2[kWaves];
-  uint32_t red_t[kWaves];
-  uint32_t red_p[kWaves];
-  float red_s[kWaves];
+  float red_f[kW];
+  uint32_t red_u[kW];
+  uint32_t red_u2[kW];
+  uint32_t red_t[kW];
+  uint32_t red_p[kW];
+  float red_s[kW];
 };
 
-struct HeadShared : Red {
+// The head's workgroup: eight waves per row, so that a row of 128 candidates
+// of 1152 bytes is in flight at once (one workgroup a compute unit at 256 rows).
+constexpr int kHeadThreads = 512;
+constexpr int kHeadWaves = kHeadThreads / kWave;
+
+struct HeadShared : Red<kHeadWaves> {
   float sc[kHeadChunkMax];  // fast score g
   float bd[kHeadChunkMax];  // bound b
   uint32_t tk[kHeadChunkMax];
@@ -385,19 +391,8 @@ struct HeadShared : Red {
   Record rec;
 };
 
-__device__ __forceinline__ float block_max(Red& sh, float v) {
-  v = wave_max(v);
-  const int w = threadIdx.x / kWave;
-  __syncthreads();
-  if ((threadIdx.x % kWave) == 0) sh.red_f[w] = v;
-  __syncthreads();
-  float out = sh.red_f[0];
-#pragma unroll
-  for (int i = 1; i < kWaves; ++i) out = __builtin_fmaxf(out, sh.red_f[i]);
-  return out;
-}
-
-__device__ __forceinline__ uint32_t block_sum(Red& sh, uint32_t v) {
+template <int kW>
+__device__ __forceinline__ uint32_t block_sum(Red<kW>& sh, uint32_t v) {
   v = wave_sum_u32(v);
   const int w = threadIdx.x / kWave;
   __syncthreads();
@@ -405,11 +400,12 @@ __device__ __forceinline__ uint32_t block_sum(Red& sh, uint32_t v) {
   __syncthreads();
   uint32_t out = 0;
 #pragma unroll
-  for (int i = 0; i < kWaves; ++i) out += sh.red_u[i];
+  for (int i = 0; i < kW; ++i) out += sh.red_u[i];
   return out;
 }
 
-__device__ __forceinline__ Best block_best(Red& sh, Best b) {
+template <int kW>
+__device__ __forceinline__ Best block_best(Red<kW>& sh, Best b) {
   b = wave_best(b);
   const int w = threadIdx.x / kWave;
   __syncthreads();
@@ -421,13 +417,14 @@ __device__ __forceinline__ Best block_best(Red& sh, Best b) {
   __syncthreads();
   Best out{sh.red_s[0], sh.red_t[0], sh.red_p[0]};
 #pragma unroll
-  for (int i = 1; i < kWaves; ++i) {
+  for (int i = 1; i < kW; ++i) {
     out = best_of(out, Best{sh.red_s[i], sh.red_t[i], sh.red_p[i]});
   }
   return out;
 }
 
-__device__ __forceinline__ void block_min_token(Red& sh, uint32_t& t,
+template <int kW>
+__device__ __forceinline__ void block_min_token(Red<kW>& sh, uint32_t& t,
                                                 uint32_t& p) {
   wave_min_token(t, p);
   const int w = threadIdx.x / kWave;
@@ -440,7 +437,39 @@ __device__ __forceinline__ void block_min_token(Red& sh, uint32_t& t,
   t = sh.red_u2[0];
   p = sh.red_p[0];
 #pragma unroll
-  for (int i = 1; i < kWaves; ++i) {
+  for (int i = 1; i < kW; ++i) {
+    if (sh.red_u2[i] < t) {
+      t = sh.red_u2[i];
+      p = sh.red_p[i];
+    }
+  }
+}
+
+// Over the workgroup, in one exchange: whether any `flag` is set, the largest
+// lo, the lowest token and its first position.
+template <int kW>
+__device__ __forceinline__ void block_bounds(Red<kW>& sh, uint32_t& flag, float& lo, uint32_t& t,
+                                             uint32_t& p) {
+  flag = __ballot(flag != 0u) != 0ull ? 1u : 0u;
+  lo = wave_max(lo);
+  wave_min_token(t, p);
+  const int w = threadIdx.x / kWave;
+  __syncthreads();
+  if ((threadIdx.x % kWave) == 0) {
+    sh.red_u[w] = flag;
+    sh.red_f[w] = lo;
+    sh.red_u2[w] = t;
+    sh.red_p[w] = p;
+  }
+  __syncthreads();
+  flag = sh.red_u[0];
+  lo = sh.red_f[0];
+  t = sh.red_u2[0];
+  p = sh.red_p[0];
+#pragma unroll
+  for (int i = 1; i < kW; ++i) {
+    flag |= sh.red_u[i];
+    lo = __builtin_fmaxf(lo, sh.red_f[i]);
     if (sh.red_u2[i] < t) {
       t = sh.red_u2[i];
       p = sh.red_p[i];
@@ -461,7 +490,7 @@ template <int H, int G, int U>
 __device__ void fast_scores_vec(const HeadArgs& a, const float* ys,
                                 HeadShared& sh, uint32_t n) {
   constexpr int L = H / (8 * G);
-  constexpr int kGroups = kThreads / G;
+  constexpr int kGroups = kHeadThreads / G;
   static_assert(L * 8 * G == H, "H must split into 16-byte lane slices");
   const int lane = threadIdx.x % G;
   const int grp = threadIdx.x / G;
@@ -512,12 +541,60 @@ __device__ void fast_scores_vec(const HeadArgs& a, const float* ys,
   }
 }
 
+// Fast scores for any H of whole 16-byte words: a wave takes U candidates at
+// a time, each lane every 64th word of each row (contiguous reads, U loads in
+// flight beside the hidden row's words from LDS).
+template <int U>
+__device__ void fast_scores_words(const HeadArgs& a, const float* ys, HeadShared& sh, uint32_t n) {
+  const uint32_t lane = threadIdx.x % kWave;
+  const uint32_t w = threadIdx.x / kWave;
+  const uint32_t words = a.H / 8u;
+  for (uint32_t base = w * U; base < n; base += kHeadWaves * U) {
+    const uint4* row[U];
+    float acc[U];
+    float acca[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {  // past the end: the last candidate again
+      const uint32_t c = base + u < n ? base + u : n - 1u;
+      row[u] = reinterpret_cast<const uint4*>(a.emb + static_cast<uint64_t>(sh.tk[c]) * a.H);
+      acc[u] = 0.0f;
+      acca[u] = 0.0f;
+    }
+    for (uint32_t q = lane; q < words; q += kWave) {
+      uint4 ev[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) ev[u] = row[u][q];
+      const float4 y0 = reinterpret_cast<const float4*>(ys)[2u * q];
+      const float4 y1 = reinterpret_cast<const float4*>(ys)[2u * q + 1u];
+      const float yv[8] = {y0.x, y0.y, y0.z, y0.w, y1.x, y1.y, y1.z, y1.w};
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const float e = half_lane(ev[u], k);
+          acc[u] = __builtin_fmaf(e, yv[k], acc[u]);
+          acca[u] = __builtin_fmaf(__builtin_fabsf(e), __builtin_fabsf(yv[k]), acca[u]);
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float g = wave_sum_f32(acc[u]);
+      const float m = wave_sum_f32(acca[u]);
+      if (lane == 0 && base + u < n) {
+        sh.sc[base + u] = g;
+        sh.bd[base + u] = __builtin_fmaf(a.coef, m, a.slack);
+      }
+    }
+  }
+}
+
 // Fast scores for any H: one wave per candidate, element-strided.
 template <typename Y>
 __device__ void fast_scores_generic(const HeadArgs& a, Y ys, HeadShared& sh, uint32_t n) {
   const int lane = threadIdx.x % kWave;
   const int w = threadIdx.x / kWave;
-  for (uint32_t c = w; c < n; c += kWaves) {
+  for (uint32_t c = w; c < n; c += kHeadWaves) {
     const uint16_t* row = a.emb + static_cast<uint64_t>(sh.tk[c]) * a.H;
     float acc = 0.0f;
     float acca = 0.0f;
@@ -541,7 +618,9 @@ __device__ void fast_scores_generic(const HeadArgs& a, Y ys, HeadShared& sh, uin
 template <int kH, int kG, typename Y>
 __device__ void fast_scores(const HeadArgs& a, Y ys, HeadShared& sh, uint32_t n) {
   if constexpr (kH > 0) {
-    fast_scores_vec<kH, kG, 2>(a, ys, sh, n);
+    fast_scores_vec<kH, kG, 1>(a, ys, sh, n);
+  } else if constexpr (kG == 8) {
+    fast_scores_words<4>(a, ys, sh, n);
   } else {
     fast_scores_generic(a, ys, sh, n);
   }
@@ -566,7 +645,7 @@ __device__ void summarize_block(const HeadArgs& a, Y ys, HeadShared& sh, uint32_
   float lo = -__builtin_huge_valf();
   uint32_t mt = kInvalidToken;
   uint32_t mp = 0u;
-  for (uint32_t c = tid; c < n; c += kThreads) {
+  for (uint32_t c = tid; c < n; c += kHeadThreads) {
     const float g = sh.sc[c];
     const float b = sh.bd[c];
     const bool ok = __builtin_isfinite(g) && __builtin_isfinite(b) && b < 0x1p100f;
@@ -577,13 +656,14 @@ __device__ void summarize_block(const HeadArgs& a, Y ys, HeadShared& sh, uint32_
       mp = pos0 + c;
     }
   }
-  const uint32_t all_finite = block_sum(sh, finite ^ 1u) == 0u;
-  const float L = block_max(sh, lo);
-  block_min_token(sh, mt, mp);
+  uint32_t bad = finite ^ 1u;
+  block_bounds(sh, bad, lo, mt, mp);
+  const bool all_finite = bad == 0u;
+  const float L = lo;
   if (tid == 0) sh.n_members = 0u;
   __syncthreads();
   // pass 2: the window {g + b >= L}; everything when not all finite
-  for (uint32_t c = tid; c < n; c += kThreads) {
+  for (uint32_t c = tid; c < n; c += kHeadThreads) {
     const bool member = !all_finite || (sh.sc[c] + sh.bd[c] >= L);
     if (member) {
       const uint32_t slot = atomicAdd(&sh.n_members, 1u);
@@ -604,7 +684,7 @@ __device__ void summarize_block(const HeadArgs& a, Y ys, HeadShared& sh, uint32_
   }
   // ambiguous window (or non-finite inputs): reference-order rescore
   Best best = best_identity();
-  for (uint32_t i = tid; i < nm; i += kThreads) {
+  for (uint32_t i = tid; i < nm; i += kHeadThreads) {
     const uint32_t c = sh.members[i];
     const uint32_t t = sh.tk[c];
     const float s = canonical_dot_order(a.order, ys, a.emb + static_cast<uint64_t>(t) * a.H, a.H);
@@ -627,7 +707,8 @@ __device__ void summarize_block(const HeadArgs& a, Y ys, HeadShared& sh, uint32_
 // otherwise the exact best (reference-order score) of the records whose
 // window reaches the best lower bound L (fast records rescored), or "all
 // NaN" when none has a finite score; the lowest id of all of them rides
-// along.  Merging in stages gives the same record as merging all at once:
+// along.  A fast record that is alone in the window stays as it is: its
+// candidate is the winner, whatever its reference-order score.  Merging in stages gives the same record as merging all at once:
 // L never exceeds the row's best exact score, so no stage drops the winner.
 // All threads must call; every thread gets the record.
 template <typename Y>
@@ -637,7 +718,7 @@ __device__ __forceinline__ Record merge_records(const HeadArgs& a, Y ys, HeadSha
   float lo = -__builtin_huge_valf();
   uint32_t mt = kInvalidToken;
   uint32_t mp = 0u;
-  for (uint32_t i = tid; i < n; i += kThreads) {
+  for (uint32_t i = tid; i < n; i += kHeadThreads) {
     const Record& q = sh.recs[i];
     inv |= (q.kind & kRecInvalid) ? 1u : 0u;
     if (q.kind & (kRecFast | kRecExact)) lo = __builtin_fmaxf(lo, q.lower);
@@ -646,13 +727,27 @@ __device__ __forceinline__ Record merge_records(const HeadArgs& a, Y ys, HeadSha
       mp = q.min_pos;
     }
   }
-  const bool invalid = block_sum(sh, inv) != 0u;
-  const float L = block_max(sh, lo);
-  block_min_token(sh, mt, mp);
+  block_bounds(sh, inv, lo, mt, mp);
+  const bool invalid = inv != 0u;
+  const float L = lo;
   const float nan = __builtin_nanf("");
   if (invalid) return Record{nan, nan, nan, kInvalidToken, 0u, kRecInvalid, mt, mp};
+  uint32_t in_window = 0u;
+  for (uint32_t i = tid; i < n; i += kHeadThreads) {
+    const Record& q = sh.recs[i];
+    if ((q.kind & (kRecFast | kRecExact)) && q.upper >= L) {
+      ++in_window;
+      sh.rec = q;  // read back only if it is the only one
+    }
+  }
+  if (block_sum(sh, in_window) == 1u) {
+    Record m = sh.rec;
+    m.min_token = mt;
+    m.min_pos = mp;
+    return m;
+  }
   Best best = best_identity();
-  for (uint32_t i = tid; i < n; i += kThreads) {
+  for (uint32_t i = tid; i < n; i += kHeadThreads) {
     const Record& q = sh.recs[i];
     if ((q.kind & (kRecFast | kRecExact)) && q.upper >= L) {
       const float s = (q.kind & kRecExact)
@@ -670,17 +765,25 @@ __device__ __forceinline__ Record merge_records(const HeadArgs& a, Y ys, HeadSha
 // Merges the row's records (sh.recs[0, n)) and writes its outputs.
 template <typename Y>
 __device__ __forceinline__ void finalize_row(const HeadArgs& a, uint32_t r, Y ys, HeadShared& sh, uint32_t n) {
-  const Record m = merge_records(a, ys, sh, n);
+  const Record m = n == 1u ? sh.recs[0] : merge_records(a, ys, sh, n);
   if (threadIdx.x == 0) {
     uint32_t token = kInvalidToken;
     float score = __builtin_nanf("");
     if (m.kind & kRecExact) {
       token = m.token;
       score = m.value;
+    } else if (m.kind & kRecFast) {
+      // (the reference-order score, a chain of H steps, only where it is asked for)
+      token = m.token;
+      if (a.out_score != nullptr) {
+        score = canonical_dot_order(a.order, ys, a.emb + static_cast<uint64_t>(m.token) * a.H, a.H);
+      }
     } else if (m.kind & kRecAllNan) {
       // every score NaN: the lowest id (greedy.cu:205-207)
       token = m.min_token;
-      score = canonical_dot_order(a.order, ys, a.emb + static_cast<uint64_t>(m.min_token) * a.H, a.H);
+      if (a.out_score != nullptr) {
+        score = canonical_dot_order(a.order, ys, a.emb + static_cast<uint64_t>(m.min_token) * a.H, a.H);
+      }
     }
     a.out_token[r] = token;
     if (a.out_score != nullptr) a.out_score[r] = score;
@@ -689,28 +792,39 @@ __device__ __forceinline__ void finalize_row(const HeadArgs& a, uint32_t r, Y ys
 
 // Loads the ids of candidates [begin, begin + n) into sh.tk; returns whether
 // any id is outside the vocabulary (the reference marks the row invalid).
-__device__ bool load_block_ids(const HeadArgs& a, const RowList& rl,
-                               HeadShared& sh, uint32_t begin, uint32_t n) {
+// first_id: entry threadIdx.x of the list, already loaded.
+__device__ bool load_block_ids(const HeadArgs& a, const RowList& rl, HeadShared& sh,
+                               uint32_t begin, uint32_t n, uint32_t first_id) {
   uint32_t bad = 0u;
-  for (uint32_t c = threadIdx.x; c < n; c += kThreads) {
-    const uint32_t t = rl.ids[begin + c];
+  for (uint32_t c = threadIdx.x; c < n; c += kHeadThreads) {
+    const uint32_t t = begin + c == threadIdx.x ? first_id : rl.ids[begin + c];
     bad |= t >= a.V ? 1u : 0u;
     sh.tk[c] = t < a.V ? t : 0u;
   }
   return block_sum(sh, bad) != 0u;
 }
 
-// One workgroup per row: the row's candidates in blocks of a.chunk, each
-// block summarized into a record in LDS, then merged (finalize_row); when
+// One workgroup per row.  Bound: latency (count and ids, candidate rows,
+// three exchanges between the waves), and at wide rows the candidate rows'
+// bytes.  A winner alone in its window needs no reference-order score (the
+// operator returns tokens), which was a chain of H steps over single global
+// loads by one thread.  256 rows of up to 128 candidates at H = 576: 13.7 -> 10.7
+// us; 200 rows of up to 128 at H = 960 154 -> 18.7, 256 rows of up to 512 at
+// H = 2048 1753 -> 117 (whole words instead of 2-byte loads).  The row's
+// candidates come in blocks of a.chunk, each block summarized into a record in LDS, then merged (finalize_row); when
 // the records fill their LDS array, they are merged into its first entry
 // and the row goes on (lists of any length).  kGlobalHidden: the hidden row
 // is read from global memory in place of an FP32 copy in LDS (rows too wide
 // for LDS).
 template <int kH, int kG, bool kGlobalHidden>
-__global__ __launch_bounds__(kThreads) void head_kernel(HeadArgs a) {
+__global__ __launch_bounds__(kHeadThreads) void head_kernel(HeadArgs a) {
   extern __shared__ __align__(16) float ys_lds[];
   __shared__ HeadShared sh;
   const uint32_t r = blockIdx.x;
+  // the list's first ids beside its count (entries of the row's fixed width)
+  const uint32_t first_id =
+      a.fixed_ids[static_cast<uint64_t>(r) * a.max_allowed +
+                  (threadIdx.x < a.max_allowed ? threadIdx.x : a.max_allowed - 1u)];
   const RowList rl = resolve_row(a, r);
   if (rl.status == 1) {
     if (threadIdx.x == 0) {
@@ -725,7 +839,7 @@ __global__ __launch_bounds__(kThreads) void head_kernel(HeadArgs a) {
     for (uint32_t blk = 0; blk < nblocks; ++blk) {
       const uint32_t begin = blk * a.chunk;
       const uint32_t n = rl.count - begin < a.chunk ? rl.count - begin : a.chunk;
-      const bool invalid = load_block_ids(a, rl, sh, begin, n);
+      const bool invalid = load_block_ids(a, rl, sh, begin, n, first_id);
       if (!invalid) fast_scores<kH, kG>(a, ys, sh, n);
       __syncthreads();
       summarize_block(a, ys, sh, n, begin, invalid);
@@ -745,8 +859,16 @@ __global__ __launch_bounds__(kThreads) void head_kernel(HeadArgs a) {
   if constexpr (kGlobalHidden) {
     body(HalfRow{a.hidden16 + static_cast<uint64_t>(r) * a.H});
   } else {
-    for (uint32_t f = threadIdx.x; f < a.H; f += kThreads) {
-      ys_lds[f] = half_to_float(a.hidden16[static_cast<uint64_t>(r) * a.H + f]);
+    const uint16_t* hidden = a.hidden16 + static_cast<uint64_t>(r) * a.H;
+    if (a.H % 8u == 0u && (reinterpret_cast<uintptr_t>(a.hidden16) & 15u) == 0u) {
+      for (uint32_t q = threadIdx.x; q < a.H / 8u; q += kHeadThreads) {
+        const uint4 h = reinterpret_cast<const uint4*>(hidden)[q];
+        float4* to = reinterpret_cast<float4*>(ys_lds) + 2u * q;
+        to[0] = float4{half_lane(h, 0), half_lane(h, 1), half_lane(h, 2), half_lane(h, 3)};
+        to[1] = float4{half_lane(h, 4), half_lane(h, 5), half_lane(h, 6), half_lane(h, 7)};
+      }
+    } else {
+      for (uint32_t f = threadIdx.x; f < a.H; f += kHeadThreads) ys_lds[f] = half_to_float(hidden[f]);
     }
     __syncthreads();
     body(static_cast<const float*>(ys_lds));
@@ -897,7 +1019,7 @@ __global__ __launch_bounds__(kThreads) void restricted_greedy_kernel(
     const void* __restrict__ logits, const uint32_t* __restrict__ allowed,
     const uint32_t* __restrict__ counts, uint32_t* __restrict__ tokens,
     uint32_t V, uint32_t max_allowed) {
-  __shared__ Red sh;
+  __shared__ Red<kWaves> sh;
   const uint32_t r = blockIdx.x;
   const uint32_t count = counts[r];
   const bool row_invalid = count == 0 || count > max_allowed;
@@ -1057,11 +1179,13 @@ hipError_t launch_head(const HeadArgs& args, hipStream_t stream) {
   const bool aligned = (reinterpret_cast<uintptr_t>(args.emb) & 15u) == 0;
   const size_t lds = static_cast<size_t>(args.H) * sizeof(float);
   if (args.H == 576 && aligned) {
-    hipLaunchKernelGGL((head_kernel<576, 8, false>), dim3(args.rows), dim3(kThreads), lds, stream, args);
+    hipLaunchKernelGGL((head_kernel<576, 8, false>), dim3(args.rows), dim3(kHeadThreads), lds, stream, args);
+  } else if (args.H % 8u == 0 && aligned && args.H <= kHeadLdsHidden) {
+    hipLaunchKernelGGL((head_kernel<0, 8, false>), dim3(args.rows), dim3(kHeadThreads), lds, stream, args);
   } else if (args.H <= kHeadLdsHidden) {
-    hipLaunchKernelGGL((head_kernel<0, 64, false>), dim3(args.rows), dim3(kThreads), lds, stream, args);
+    hipLaunchKernelGGL((head_kernel<0, 64, false>), dim3(args.rows), dim3(kHeadThreads), lds, stream, args);
   } else {
-    hipLaunchKernelGGL((head_kernel<0, 64, true>), dim3(args.rows), dim3(kThreads), 0, stream, args);
+    hipLaunchKernelGGL((head_kernel<0, 64, true>), dim3(args.rows), dim3(kHeadThreads), 0, stream, args);
   }
   return hipGetLastError();
 }

@@ -125,3 +125,34 @@ def test_stream_head_tiles_match_the_oracle(rows, open_rows, vocab, hidden):
     assert w.unrestricted_rows.size == open_rows
     assert np.array_equal(tok, etok) and np.array_equal(nx, enx)
     assert np.array_equal(sc.view(np.uint32), esc.view(np.uint32))
+
+
+@pytest.mark.parametrize("hidden", [8, 520, 576, 960, 2048, 100])
+@pytest.mark.parametrize("width", [1, 3, 128, 129, 515])
+def test_head_words_blocks_and_ties(hidden, width):
+    """Rows of whole words and not, lists of one block, one candidate more and
+    several; equal table rows (the lower id wins), NaN and infinite rows, an
+    all-NaN list, a list with an id past the vocabulary and empty ones."""
+    from market_sim_amd import ops
+    rng = np.random.default_rng(hidden + width)
+    rows, vocab = 9, 1200
+    h = rng.standard_normal((rows, hidden)).astype(np.float16)
+    e = (rng.standard_normal((vocab, hidden)) * 0.05).astype(np.float16)
+    e[600:1200] = e[0:600]              # every score twice
+    e[5, hidden // 2] = np.nan
+    e[7, 0] = np.inf
+    e[40:60] = np.nan
+    allowed = np.stack([rng.permutation(vocab)[:width] for _ in range(rows)]).astype(np.uint32)
+    counts = rng.integers(1, width + 1, rows).astype(np.uint32)
+    counts[0] = width
+    counts[1] = 0
+    counts[2] = width + 1
+    allowed[3, :] = 40 + np.arange(width) % 20
+    allowed[4, counts[4] - 1] = vocab
+    hb, eb = h.view(np.uint16), e.view(np.uint16)
+    out = empty(rows, np.uint32)
+    keep = [dev(x) for x in (hb, eb, allowed, counts)]
+    ok(ops.restricted_output_head_f16(*[B(t) for t in keep], B(out), rows, hidden, vocab, width,
+                                      stream()))
+    want, _ = oracle.restricted_output_head_f16(hb, eb, allowed, counts, width)
+    assert host(out, np.uint32).tolist() == want.tolist()
