@@ -482,20 +482,35 @@ bool optional_is(const mf_buffer& b, uint64_t bytes) {
 // MFMA step (64-candidate wave tiles); otherwise on the VALU dot.
 bool mfma_gather(uint64_t H) { return H % 32u == 0; }
 // Candidates per gather tile (one wave each on the MFMA gather).  Tiles of
-// 64 unless the pack is small: when even the upper bound of its 64-candidate
-// tiles (every row as long as the longest list) stays under four per
-// compute unit of an MI355X (256 CUs), a wave would stream 64 rows through
-// eight dependent load units while most SIMDs idle, so the tiles shrink to
-// 32 or 16 candidates (more waves, one or two units each; the finalize
-// merges the extra records).
+// 64 unless the pack is small: with fewer than four 64-candidate tiles per
+// compute unit of an MI355X (256 CUs) a wave would stream 64 rows through
+// dependent load units while most SIMDs idle, so the tiles shrink to 32 or 16
+// candidates (more waves, one or two units each; the finalize merges the extra
+// records).  The pack's candidates are counted as rows times the states' mean
+// list (rows times the longest list, the upper bound, took 97 rows of lists up
+// to 2048 for eight times what they hold: gather 14.7 -> 11.7 us at H = 960
+// with tiles of 16; 64 rows at H = 576, the step 34.3 -> 32.5; 250 rows of up to
+// 4096, 1700 tiles of 64, lose with 16: 48.3 against 49.2).  The records are laid
+// out for the longest list, so the tiles shrink only while those stay few.
+// bound: the tile by that upper bound, which the layout falls back to.
 constexpr uint64_t kGatherSmallPack = 4u * 256u;
-uint32_t gather_tile(uint64_t H, uint64_t rows, uint64_t max_count) {
-  if (!mfma_gather(H)) return H == 2048 ? 128u : 64u;
-  const uint64_t lists = max_count == 0 ? 1 : max_count;
-  const uint64_t t64 = rows * ((lists + mf::kGatherWaveTile - 1) / mf::kGatherWaveTile);
-  if (t64 >= kGatherSmallPack) return mf::kGatherWaveTile;
-  const uint64_t t32 = rows * ((lists + 31) / 32);
-  return t32 >= kGatherSmallPack ? 32u : 16u;
+constexpr uint64_t kGatherRecordsMax = 1u << 16;
+uint32_t gather_tile(const mf_decode_tail_args* a, bool bound) {
+  if (!mfma_gather(a->hidden)) return a->hidden == 2048 ? 128u : 64u;
+  const uint64_t longest = a->max_count == 0 ? 1 : a->max_count;
+  auto tiles = [a](uint64_t list, uint64_t tile) { return a->rows * ((list + tile - 1u) / tile); };
+  uint32_t tile = mf::kGatherWaveTile;
+  if (bound) {
+    while (tile > 16u && tiles(longest, tile) < kGatherSmallPack) tile /= 2u;
+    return tile;
+  }
+  const uint64_t mean = (a->nnz + a->states - 1) / a->states;
+  while (tile > 16u && a->rows * (mean < longest ? mean : longest) / tile < kGatherSmallPack &&
+         tiles(longest, tile / 2u) <= kGatherRecordsMax) {
+    tile /= 2u;
+  }
+  const uint32_t least = gather_tile(a, true);
+  return tile < least ? tile : least;
 }
 
 // The table pass (one launch for restricted and unrestricted rows): lists
@@ -646,14 +661,17 @@ mf_status validate_tail(const mf_decode_tail_args* a, bool full, TailLayout& L) 
     return status(MF_INVALID_ARGUMENT);
   }
   const uint64_t rows = a->rows;
+  auto list_tiles = [a](uint32_t tile) {
+    return static_cast<uint32_t>(a->max_count == 0 ? 1 : (a->max_count + tile - 1) / tile);
+  };
   if (full) {
     // unrestricted rows take the whole vocabulary as their list
     const uint64_t longest = a->max_count > a->vocab ? a->max_count : a->vocab;
     L.tile = kFullTile;
     L.max_tiles = static_cast<uint32_t>((longest + L.tile - 1) / L.tile);
   } else {
-    L.tile = gather_tile(a->hidden, a->rows, a->max_count);
-    L.max_tiles = static_cast<uint32_t>(a->max_count == 0 ? 1 : (a->max_count + L.tile - 1) / L.tile);
+    L.tile = gather_tile(a, true);
+    L.max_tiles = list_tiles(L.tile);
   }
   // table pass: one record per (row, 192-token range) holding its ids
   L.pass = !full && table_pass(a);
@@ -710,18 +728,26 @@ mf_status validate_tail(const mf_decode_tail_args* a, bool full, TailLayout& L) 
     L.dense_flag = take(L.dense ? rows * 4u : 0u);
     L.total = off;
   };
-  place();
-  if (!L.pass && !L.dense && fb_rows > 0) {
-    // the stream head's tiles: as fine as its compute units want, or coarse
-    // when only that keeps the workspace within the no-allocation array
-    for (const bool coarse : {true, false}) {
-      const TailLayout before = L;
+  // The gather's tiles and the stream head's: first as coarse as the upper
+  // bound of the pack and the table pass's tiles make them, then as fine as
+  // the compute units want, unless only the coarse ones keep the workspace
+  // within the no-allocation array.
+  const bool stream = !full && !L.pass && !L.dense && fb_rows > 0;
+  auto with_tiles = [&](bool coarse) {
+    if (!full && !L.pass) {
+      L.tile = gather_tile(a, coarse);
+      L.max_tiles = list_tiles(L.tile);
+    }
+    if (stream) {
       L.fb_blocks = mf::stream_tile_blocks(vocab, coarse);
       L.fb_tiles = mf::stream_tiles(vocab, L.fb_blocks);
-      place();
-      if (!coarse && before.total <= kScratchBytes && L.total > kScratchBytes) L = before;
     }
-  }
+    place();
+  };
+  with_tiles(true);
+  const TailLayout coarse = L;
+  with_tiles(false);
+  if (coarse.total <= kScratchBytes && L.total > kScratchBytes) L = coarse;
   return ok();
 }
 
