@@ -10,22 +10,28 @@
 // work instead (2 H flops per slot and token).
 //
 // Workgroup: a panel of 256 slots (16 blocks of 16) x one tile of 12 token
-// blocks, eight waves.  MFMA wave w (0-3) takes the row blocks of parity
-// w % 2 and the six token blocks of half w / 2 (8 x 6 MFMA blocks,
-// v_mfma_f32_16x16x32_f16); waves 4-7 issue the copies (a wave issuing
+// blocks, twelve waves.  Eight MFMA waves, two a SIMD, so that one's MFMAs run
+// under the other's LDS reads: wave w (0-7) takes the row blocks 4 i + w % 4
+// and the six token blocks of half w / 4 (4 x 6 MFMA blocks,
+// v_mfma_f32_16x16x32_f16); waves 8-11 issue the copies (a wave issuing
 // copies stalls while the address unit is busy, and an MFMA wave would idle
-// with it).  K runs in 32-feature steps; each step's A rows (the slots' FP16
-// hi of z = x * w, from L2) and B rows (the tile's table rows, from HBM) are
-// copied straight into LDS (global_load_lds, 16 bytes per lane), three steps
-// in flight beside the one being multiplied; one barrier per step hands it
-// over.  LDS rows are 64 bytes; piece p of row r sits at p ^ swz(r), so the
-// 16 rows one fragment read touches fall on distinct banks.  The MFMA waves
-// also sum the squares of the table fragments they read (FP32, any order),
-// which gives the token norms of the bounds.
+// with it).  K runs in chunks of 64 features (whole 128-byte lines): a chunk's
+// A rows (the slots' FP16 hi of z = x * w, from L2) in four units of 64 rows
+// and its B rows (the tile's table rows, from HBM) are copied straight into LDS
+// (global_load_lds, 16 bytes per lane), into rings of two chunks and a unit
+// and of three chunks; one barrier per chunk, where every MFMA wave has its
+// last fragments in registers.  The 16-byte pieces of a row are XOR-swizzled
+// by the row's bits 1-3, so the 16 lanes one read cycle serves meet 16 bank
+// groups.  The MFMA waves also sum the squares of the table fragments they read
+// (FP32, any order), which gives the token norms of the bounds.
+// One panel (51 open and 205 listed rows) at H = 2048, V = 128256, three
+// tiles on most compute units: 198 -> 174 us (from 32-feature steps, 64 bytes a
+// row, in four MFMA waves); bound by the copies as the projection GEMM (1.4 us a
+// chunk) and by the epilogue and first copies of each tile, about 14 us.
 //
 // Epilogue per tile: the slot's allowed tokens of the tile come from the
 // norm launch's span index (a 192-bit mask and the list position of the
-// first id), copied into LDS during the previous tile; per slot the best
+// first id), copied into LDS ahead of the tile's chunks; per slot the best
 // lower bound over allowed tokens, the members (fl(g + b) >= L) and one
 // TileRecord in the MFMA head's format (list positions for restricted rows,
 // token ids for unrestricted ones).
@@ -47,32 +53,42 @@ namespace {
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-constexpr int kMmaWaves = 4;
+constexpr int kMmaWaves = 8;
 constexpr int kCopyWaves = 4;
 constexpr int kWaves = kMmaWaves + kCopyWaves;
 constexpr int kThreads = kWaves * kWave;
-static_assert(kMmaWaves * kWave == static_cast<int>(kDensePanelSlots), "one MFMA thread per slot");
-constexpr int kRBw = 8;  // row blocks per MFMA wave
-constexpr int kTBw = 6;  // token blocks per MFMA wave
-constexpr int kNormBw = 3;  // token blocks whose norms the MFMA wave forms
-constexpr int kStages = 4;
-constexpr uint32_t kABytes = kDensePanelSlots * 64u;  // one 32-feature step of every slot
-constexpr uint32_t kBBytes = kHeadTileTokens * 64u;   // one step of the tile's table rows
-constexpr uint32_t kStageBytes = kABytes + kBBytes;
-constexpr int kADma = static_cast<int>(kABytes / 1024u / kCopyWaves);  // 1 KiB copies per wave
-constexpr int kBDma = static_cast<int>(kBBytes / 1024u / kCopyWaves);
-constexpr int kDmaPerWave = kADma + kBDma;
-static_assert(kADma == 4 && kBDma == 3, "copy split");
-// epilogue rows in the stage area: [slot][33] arrays of the lanes' values
+constexpr int kRBw = 4;     // row blocks per MFMA wave
+constexpr int kTBw = 6;     // token blocks per MFMA wave
+constexpr int kNormBw = 2;  // token blocks whose norms an MFMA wave forms, at most
+constexpr uint32_t kKC = 64;          // features per chunk
+constexpr uint32_t kRow = kKC * 2u;   // bytes of a row in a chunk
+// the rings: A rows in units of 64 (one row block of each MFMA wave), two
+// chunks and a unit; the tile's table rows, three chunks
+constexpr uint32_t kAUnits = 4;
+constexpr uint32_t kASlots = 2u * kAUnits + 1u;
+constexpr uint32_t kAUnitRows = kDensePanelSlots / kAUnits;
+constexpr uint32_t kAUnitBytes = kAUnitRows * kRow;
+constexpr uint32_t kBSlots = 3;
+constexpr uint32_t kBBytes = kHeadTileTokens * kRow;
+constexpr uint32_t kRingBytes = kASlots * kAUnitBytes + kBSlots * kBBytes;
+constexpr int kACopies = static_cast<int>(kAUnitBytes / 1024u / kCopyWaves);  // 1 KiB copies per wave
+constexpr int kBCopies = static_cast<int>(kBBytes / 1024u / kCopyWaves);
+static_assert(kACopies == 2 && kBCopies == 6, "copy split");
+// copies per wave: what is brought ahead of the chunk before (a unit of A,
+// the table rows), and the rest of a chunk
+constexpr int kAhead = kACopies + kBCopies;
+constexpr int kRest = static_cast<int>(kAUnits - 1u) * kACopies;
+// epilogue rows in the rings' area: [slot][33] arrays of the lanes' values
 // (two of floats, one of bytes), then the tile's records staged for the
 // store
 constexpr uint32_t kEpiRow = 33;
 constexpr uint32_t kEpiRowsBytes = kDensePanelSlots * kEpiRow * 4u;
 constexpr uint32_t kEpiBlockBytes = (kDensePanelSlots * kEpiRow + 15u) / 16u * 16u;  // bytes
-static_assert(2u * kEpiRowsBytes + kEpiBlockBytes + kDensePanelSlots * 96u <=
-                  kStages * kStageBytes,
-              "epilogue rows and staged records in the stages");
-static_assert(kMmaWaves * kTBw / 2 == static_cast<int>(kHeadTileTokens / 16u), "tile");
+static_assert(2u * kEpiRowsBytes + kEpiBlockBytes + kDensePanelSlots * 96u <= kRingBytes,
+              "epilogue rows and staged records in the rings");
+static_assert(2 * kTBw == static_cast<int>(kHeadTileTokens / 16u) &&
+                  4 * kRBw * 16 == static_cast<int>(kDensePanelSlots),
+              "tile and panel");
 
 enum : uint32_t { kSlotNone = 0u, kSlotAll = 1u, kSlotList = 2u };
 
@@ -81,16 +97,21 @@ struct DenseShared {
   float slot_norm[kDensePanelSlots];
   float slot_slack[kDensePanelSlots];
   uint32_t slot_kind[kDensePanelSlots];
-  uint4 span[2][kDensePanelSlots][2];  // per tile parity: {m0,m1,m2,lo},{m3,m4,m5,cnt}
+  uint4 span[kDensePanelSlots][2];  // {m0,m1,m2,lo},{m3,m4,m5,cnt}
   float tn[kMmaWaves];
   uint32_t wave_sum[kWaves];
 };
 
 __host__ __device__ constexpr uint32_t dense_lds_bytes() {
-  return kStages * kStageBytes + static_cast<uint32_t>(sizeof(DenseShared));
+  return kRingBytes + static_cast<uint32_t>(sizeof(DenseShared));
 }
 
-__device__ __forceinline__ uint32_t swz(uint32_t r) { return ((r >> 1) ^ (r >> 3)) & 3u; }
+static_assert(dense_lds_bytes() <= 160u * 1024u, "LDS");
+
+// LDS byte offset of piece p (0..7) of row r of a ring slot: the 16 lanes one
+// ds_read_b128 cycle serves meet 16 bank groups
+__device__ __forceinline__ uint32_t swz(uint32_t r) { return (r >> 1) & 7u; }
+__device__ __forceinline__ uint32_t piece_at(uint32_t r, uint32_t p) { return r * kRow + (p ^ swz(r)) * 16u; }
 
 // The slot list of the launch: unrestricted rows first (fb_rows order), then
 // the kRowDense rows in row order; panel p of P takes slots [p0, p0 + n)
@@ -153,10 +174,10 @@ __device__ void dense_slots(const DenseArgs& a, DenseShared& sh, uint32_t p0, ui
   __syncthreads();
 }
 
-// Wait until at most kAfter steps of this copy wave's copies are in flight.
-template <int kAfter>
-__device__ __forceinline__ void wait_steps() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAfter * kDmaPerWave) : "memory");
+// Wait until at most kN of this copy wave's copies are in flight.
+template <int kN>
+__device__ __forceinline__ void wait_copies() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kN) : "memory");
 }
 
 // A workgroup barrier without __syncthreads' release fence, which would wait
@@ -168,14 +189,14 @@ __device__ __forceinline__ void step_barrier() {
 
 __global__ __launch_bounds__(kThreads) void dense_kernel(DenseArgs a) {
   extern __shared__ __align__(16) unsigned char dyn[];
-  DenseShared& sh = *reinterpret_cast<DenseShared*>(dyn + kStages * kStageBytes);
+  DenseShared& sh = *reinterpret_cast<DenseShared*>(dyn + kRingBytes);
   const uint32_t tid = threadIdx.x;
   const uint32_t lane = tid % kWave;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const bool copier = wave >= static_cast<uint32_t>(kMmaWaves);
   const uint32_t cw = wave % kCopyWaves;  // copy wave index (copy waves)
-  const uint32_t wm = wave % 2u;  // row-block parity (MFMA waves)
-  const uint32_t wn = (wave / 2u) % 2u;  // token half (MFMA waves)
+  const uint32_t wm = wave % 4u;  // row block of each unit (MFMA waves)
+  const uint32_t wn = (wave / 4u) % 2u;  // token half (MFMA waves)
   const uint32_t col = lane % 16u;
   const uint32_t kb = lane / 16u;
   // workgroup -> (group, panel): the compute units of one XCD in groups of
@@ -209,9 +230,9 @@ __global__ __launch_bounds__(kThreads) void dense_kernel(DenseArgs a) {
   const uint32_t panel = l % P;
   const uint32_t p0 = panel * n_slots / P;
   const uint32_t pn = (panel + 1u) * n_slots / P - p0;
-  // row blocks with slots; wave parity wm takes blocks 2 i + wm, i < nact
+  // row blocks with slots; waves wm take blocks 4 i + wm, i < nact
   const uint32_t nrb = (pn + 15u) / 16u;
-  const uint32_t nact = nrb > wm ? (nrb - wm + 1u) / 2u : 0u;
+  const uint32_t nact = nrb > wm ? (nrb - wm + 3u) / 4u : 0u;
   const uint32_t grp = x * gpx + l / P;
   const uint32_t groups = xcds * gpx;
   const uint32_t tiles = a.ranges;
@@ -219,8 +240,9 @@ __global__ __launch_bounds__(kThreads) void dense_kernel(DenseArgs a) {
   const uint32_t t_end = static_cast<uint32_t>(static_cast<uint64_t>(tiles) * (grp + 1u) / groups);
   dense_slots(a, sh, p0, pn, grp == 0u);
   const uint32_t H = a.H;
-  const uint32_t steps = H / 32u;
-  // The tile's LDS epilogue areas (the stage area, free after the K loop):
+  const uint32_t chunks = (H + kKC - 1u) / kKC;
+  unsigned char* const bring = dyn + kASlots * kAUnitBytes;
+  // The tile's LDS epilogue areas (the rings, free after the K loop):
   // per-lane values of each slot in rows of 33 words (word 16 half + column
   // of slot s's row, padded so the four slots of one write sit on different
   // banks), then the tile's records, staged for the store.
@@ -244,138 +266,169 @@ __global__ __launch_bounds__(kThreads) void dense_kernel(DenseArgs a) {
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   };
-  // The copy waves: every tile's steps, then the barriers of the MFMA
+  // The copy waves: every tile's chunks, then the barriers of the MFMA
   // waves' epilogue.  (Separate loops for the two kinds of waves, so that
   // neither holds the other's registers.)
   auto copy_tiles = [&]() {
-    // per-lane copy sources of a copy wave: A rows (4 copies of 16 rows),
+    // per-lane copy sources of a copy wave: copy i of unit u brings A rows
+    // 64 u + 8 (cw + 4 i) .., lane l row l / 8 of them, LDS piece l % 8; the
     // span records (2 copies of 32 slots)
-    uint32_t aoff[kADma];
-  #pragma unroll
-    for (int j = 0; j < kADma; ++j) {
-      const uint32_t r = (cw * kADma + j) * 16u + lane / 4u;
-      aoff[j] = sh.slot_row[r] * H + (((lane % 4u) ^ swz(r)) * 8u);
+    uint32_t aoff[kAUnits][kACopies];
+#pragma unroll
+    for (uint32_t u = 0; u < kAUnits; ++u) {
+#pragma unroll
+      for (int i = 0; i < kACopies; ++i) {
+        const uint32_t r = kAUnitRows * u + 8u * (cw + kCopyWaves * i) + lane / 8u;
+        aoff[u][i] = sh.slot_row[r] * H + (((lane % 8u) ^ swz(r)) * 8u);
+      }
     }
     uint32_t srow[2];
-  #pragma unroll
+#pragma unroll
     for (int j = 0; j < 2; ++j) {
       const uint32_t s = ((cw * 2u + j) * kWave + lane) / 2u;
       srow[j] = sh.slot_kind[s] == kSlotList ? sh.slot_row[s] : 0u;
     }
-    auto issue_span = [&](uint32_t tile) {
-      uint4* dst = &sh.span[tile & 1u][0][0];
-  #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const uint32_t idx = (cw * 2u + j) * kWave + lane;
-        const uint4* src = a.spans + (static_cast<uint64_t>(tile) * a.rows + srow[j]) * 2u + (idx % 2u);
-        burst_to_lds(src, dst + (cw * 2u + j) * kWave);
-      }
-    };
-    if (t_begin < t_end) issue_span(t_begin);
+    // (rows 8 n + lane / 8 with the same lane share their swizzle up to n's
+    // parity; a piece past a last half chunk re-reads the half before)
+    const uint32_t piece0 = (lane % 8u) ^ swz(8u * cw + lane / 8u);
     for (uint32_t tile = t_begin; tile < t_end; ++tile) {
       const uint32_t tok0 = tile * kHeadTileTokens;
       const uint32_t nt = a.V - tok0 < kHeadTileTokens ? a.V - tok0 : kHeadTileTokens;
-      if (tile + 1u < t_end) issue_span(tile + 1u);
+      {
+        uint4* dst = &sh.span[0][0];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const uint32_t idx = (cw * 2u + j) * kWave + lane;
+          const uint4* src = a.spans + (static_cast<uint64_t>(tile) * a.rows + srow[j]) * 2u + (idx % 2u);
+          burst_to_lds(src, dst + (cw * 2u + j) * kWave);
+        }
+      }
       const uint16_t* tbase = a.emb + static_cast<uint64_t>(tok0) * H;
-      uint32_t boff[kBDma];
+      uint32_t boff[kBCopies];
 #pragma unroll
-      for (int j = 0; j < kBDma; ++j) {
-        const uint32_t t = (cw * kBDma + j) * 16u + lane / 4u;
+      for (int i = 0; i < kBCopies; ++i) {
+        const uint32_t t = 8u * (cw + kCopyWaves * i) + lane / 8u;
         const uint32_t tc = t < nt ? t : nt - 1u;
-        boff[j] = tc * H + (((lane % 4u) ^ swz(t)) * 8u);
+        boff[i] = tc * H + (((lane % 8u) ^ swz(t)) * 8u);
       }
-      auto issue = [&](uint32_t s) {
-        unsigned char* st = dyn + (s % kStages) * kStageBytes;
-        const uint32_t f = s * 32u;
-#pragma unroll
-        for (int j = 0; j < kADma; ++j) {
-          burst_to_lds(a.z_hi + aoff[j] + f, st + (cw * kADma + j) * 1024u);
-        }
-#pragma unroll
-        for (int j = 0; j < kBDma; ++j) {
-          burst_to_lds(tbase + boff[j] + f, st + kABytes + (cw * kBDma + j) * 1024u);
-        }
+      // the features of chunk c at this lane's pieces
+      auto feature = [&](uint32_t c) {
+        return c * kKC - (c * kKC + piece0 * 8u >= H ? 32u : 0u);
       };
-      // steps 0 .. kStages - 2 in flight; then per step s the copies of step
-      // s + kStages - 1 go into the stage of step s - 1 (every MFMA wave is
-      // done with it), and step s + 1 is handed over once it has landed.
-      // Past the last step the last one is copied again (into a stage
-      // nobody reads), so that every step issues the same copies.
+      uint32_t aslot = 0, bslot = 0;  // the next unit's and chunk's
+      auto issue_a = [&](uint32_t c, uint32_t u) {
+        unsigned char* buf = dyn + aslot * kAUnitBytes;
+        const uint32_t f = feature(c);
 #pragma unroll
-      for (int s = 0; s < kStages - 1; ++s) issue(static_cast<uint32_t>(s) < steps ? s : steps - 1u);
-      wait_steps<kStages - 2>();
-      step_barrier();  // step 0 in LDS
-      for (uint32_t s = 0; s < steps; ++s) {
-        issue(s + kStages - 1 < steps ? s + kStages - 1 : steps - 1u);
-        wait_steps<kStages - 2>();
-        step_barrier();  // step s + 1 in LDS, step s read by every MFMA wave
+        for (int i = 0; i < kACopies; ++i) {
+          const uint32_t off = u == 0u ? aoff[0][i] : (u == 1u ? aoff[1][i] : (u == 2u ? aoff[2][i] : aoff[3][i]));
+          burst_to_lds(a.z_hi + off + f, buf + (cw + kCopyWaves * i) * 1024u);
+        }
+        if (++aslot == kASlots) aslot = 0u;
+      };
+      auto issue_ahead = [&](uint32_t c) {
+        issue_a(c, 0u);
+        unsigned char* buf = bring + bslot * kBBytes;
+        const uint32_t f = feature(c);
+#pragma unroll
+        for (int i = 0; i < kBCopies; ++i) {
+          burst_to_lds(tbase + boff[i] + f, buf + (cw + kCopyWaves * i) * 1024u);
+        }
+        if (++bslot == kBSlots) bslot = 0u;
+      };
+      auto issue_rest = [&](uint32_t c) {
+        issue_a(c, 1u);
+        issue_a(c, 2u);
+        issue_a(c, 3u);
+      };
+      // two chunks and the part of a third in flight (the launcher checks
+      // that there are three); then per chunk c, once chunk c + 1 has landed and
+      // every MFMA wave has read chunk c, what its slots make room for
+      issue_ahead(0u);
+      issue_rest(0u);
+      issue_ahead(1u);
+      issue_rest(1u);
+      issue_ahead(2u);
+      wait_copies<2 * kAhead + kRest>();
+      step_barrier();  // chunk 0 in LDS
+      for (uint32_t c = 0; c < chunks; ++c) {
+        if (c + 2u < chunks) {
+          wait_copies<kAhead>();
+        } else {
+          wait_copies<0>();
+        }
+        step_barrier();  // chunk c + 1 in LDS, chunk c read by every MFMA wave
+        if (c + 2u < chunks) issue_rest(c + 2u);
+        if (c + 3u < chunks) issue_ahead(c + 3u);
       }
-      // the copies past the last step, and the span copies, have landed;
-      // then the MFMA waves' epilogue phases (the same barriers)
-      wait_vector_memory();
-      __syncthreads();
+      // the MFMA waves' epilogue phases (the same barriers)
       __syncthreads();
       __syncthreads();
       __syncthreads();
       store_records(tile);
     }
   };
-  // The MFMA waves (thread tid is slot tid), with NACT of the wave's row
-  // blocks holding slots (a variant per count, so the loop has no branch
+  // The MFMA waves (threads 0 .. 255 also stand for the panel's slots), with
+  // NACT of the wave's row blocks holding slots (a variant per count, so the loop has no branch
   // around an MFMA).
   auto mfma_tiles = [&]<int NACT>() {
     for (uint32_t tile = t_begin; tile < t_end; ++tile) {
       const uint32_t tok0 = tile * kHeadTileTokens;
       const uint32_t nt = a.V - tok0 < kHeadTileTokens ? a.V - tok0 : kHeadTileTokens;
-      const uint32_t b = tile & 1u;
-      // (the MFMA waves hold the slots: thread tid is slot tid)
       floatx4 acc[kRBw][kTBw];
 #pragma unroll
       for (int i = 0; i < kRBw; ++i) {
 #pragma unroll
         for (int j = 0; j < kTBw; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
       }
-      // per lane: the sums of squares of its features of the tokens of its
-      // three norm blocks
-      float tsq[kNormBw] = {0.0f, 0.0f, 0.0f};
-      step_barrier();  // step 0 in LDS
-      for (uint32_t s = 0; s < steps; ++s) {
-        const unsigned char* st = dyn + (s % kStages) * kStageBytes;
-        half8_t fb[kTBw];
+      // per lane: the sums of squares of its features of the tokens of the
+      // wave's norm blocks (token blocks wm, wm + 4 of its half)
+      float tsq[kNormBw] = {0.0f, 0.0f};
+      uint32_t as = 0, bs = 0;  // the slots of the chunk's first unit and table rows
+      half8_t fa[kRBw], fb[kTBw];
+      auto read_half = [&](uint32_t h) {
+        const uint32_t p = 4u * h + kb;
+        const unsigned char* bbuf = bring + bs * kBBytes;
 #pragma unroll
         for (int j = 0; j < kTBw; ++j) {
-          const uint32_t t = (wn * kTBw + j) * 16u + col;
-          fb[j] = *reinterpret_cast<const half8_t*>(st + kABytes + t * 64u + ((kb ^ swz(t)) * 16u));
-        }
-        // the row blocks' A fragments one ahead of their MFMAs
-        auto read_a = [&](int i) {
-          const uint32_t r = (2u * static_cast<uint32_t>(i) + wm) * 16u + col;
-          return *reinterpret_cast<const half8_t*>(st + r * 64u + ((kb ^ swz(r)) * 16u));
-        };
-        half8_t fa = read_a(0);
-#pragma unroll
-        for (int j = 0; j < kNormBw; ++j) {
-          const half8_t g = wm == 0u ? fb[j] : fb[kNormBw + j];  // (wm is wave-uniform)
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const float v = static_cast<float>(g[e]);
-            tsq[j] = __builtin_fmaf(v, v, tsq[j]);
-          }
+          fb[j] = *reinterpret_cast<const half8_t*>(bbuf + piece_at((wn * kTBw + j) * 16u + col, p));
         }
 #pragma unroll
         for (int i = 0; i < NACT; ++i) {
-          const half8_t fn = read_a(i + 1 < NACT ? i + 1 : i);
-          __builtin_amdgcn_sched_barrier(0);
+          const uint32_t slot = as + i < kASlots ? as + i : as + i - kASlots;
+          fa[i] = *reinterpret_cast<const half8_t*>(dyn + slot * kAUnitBytes + piece_at(16u * wm + col, p));
+        }
+      };
+      auto multiply = [&]() {
+#pragma unroll
+        for (int i = 0; i < NACT; ++i) {
 #pragma unroll
           for (int j = 0; j < kTBw; ++j) {
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa, fb[j], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[i], fb[j], acc[i][j], 0, 0, 0);
           }
-          __builtin_amdgcn_sched_barrier(0);
-          fa = fn;
         }
-        step_barrier();  // this wave is done with step s
+#pragma unroll
+        for (int j = 0; j < kTBw; ++j) {
+          if (static_cast<uint32_t>(j % 4) == wm) {  // (wave-uniform)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const float v = static_cast<float>(fb[j][e]);
+              tsq[j / 4] = __builtin_fmaf(v, v, tsq[j / 4]);
+            }
+          }
+        }
+      };
+      step_barrier();  // chunk 0 in LDS
+      for (uint32_t c = 0; c < chunks; ++c) {
+        read_half(0u);
+        multiply();
+        read_half(1u);
+        step_barrier();  // this wave's reads of chunk c have arrived
+        if ((as += kAUnits) >= kASlots) as -= kASlots;
+        if (++bs == kBSlots) bs = 0u;
+        if (c * kKC + 32u < H) multiply();
       }
-      __syncthreads();  // every copy landed
+      // (after the last barrier nothing reads or writes the rings)
 
       // token norms: lanes c, c + 16, c + 32, c + 48 hold the four K
       // quarters of column c's sum; a NaN norm (non-finite table row)
@@ -386,7 +439,7 @@ __global__ __launch_bounds__(kThreads) void dense_kernel(DenseArgs a) {
         uint32_t el = lane;
         asm volatile("" : "+v"(el));
         const uint32_t ecol = el % 16u;
-        const uint32_t t0 = (wn * kTBw + wm * kNormBw) * 16u + ecol;
+        const uint32_t t0 = (wn * kTBw + wm) * 16u + ecol;
         const int up16 = static_cast<int>((el ^ 16u) * 4u);
         const int up32 = static_cast<int>((el ^ 32u) * 4u);
         float tn_local = 0.0f;
@@ -396,8 +449,8 @@ __global__ __launch_bounds__(kThreads) void dense_kernel(DenseArgs a) {
           float q = tsq[j];
           q += __int_as_float(__builtin_amdgcn_ds_bpermute(up16, __float_as_int(q)));
           q += __int_as_float(__builtin_amdgcn_ds_bpermute(up32, __float_as_int(q)));
-          const uint32_t t = t0 + 16u * static_cast<uint32_t>(j);
-          if (el < 16u && t < nt) {
+          const uint32_t t = t0 + 64u * static_cast<uint32_t>(j);
+          if (el < 16u && t < nt && wm + 4u * static_cast<uint32_t>(j) < kTBw) {
             const float v = __fsqrt_rn(q) * (1.0f + 0x1p-7f);
             tn_nan |= v != v;
             tn_local = __builtin_fmaxf(tn_local, v);
@@ -412,7 +465,7 @@ __global__ __launch_bounds__(kThreads) void dense_kernel(DenseArgs a) {
       // (thread tid's slot index made opaque here for the same reason)
       uint32_t es = tid;
       asm volatile("" : "+v"(es));
-      {
+      if (es < kDensePanelSlots) {
         const uint32_t kind = sh.slot_kind[es];
         if (kind != kSlotList) {
           uint32_t w[6];
@@ -422,17 +475,17 @@ __global__ __launch_bounds__(kThreads) void dense_kernel(DenseArgs a) {
             w[k] = kind == kSlotNone ? 0u
                    : (nt >= lo + 32u ? 0xFFFFFFFFu : (nt > lo ? (1u << (nt - lo)) - 1u : 0u));
           }
-          sh.span[b][es][0] = uint4{w[0], w[1], w[2], tok0};
-          sh.span[b][es][1] = uint4{w[3], w[4], w[5], kind == kSlotNone ? 0u : nt};
+          sh.span[es][0] = uint4{w[0], w[1], w[2], tok0};
+          sh.span[es][1] = uint4{w[3], w[4], w[5], kind == kSlotNone ? 0u : nt};
         }
       }
       __syncthreads();
-      // lane bases: slot (i, q) of this lane is sbase + 32 i + q (opaque to
+      // lane bases: slot (i, q) of this lane is sbase + 64 i + q (opaque to
       // the compiler, so that the epilogue's addresses are formed here and not
       // hoisted out of the tile loop, where they would outlive the registers)
       uint32_t sbase = wm * 16u + 4u * kb;
       asm volatile("" : "+v"(sbase));
-      const uint4* spn = &sh.span[b][sbase][wn];
+      const uint4* spn = &sh.span[sbase][wn];
       const uint32_t sel0 = 1u << col;
       const uint32_t sel1 = 1u << (16u + col);
       const uint32_t lw = sbase * kEpiRow + wn * 16u + col;  // this lane's word of slot sbase
@@ -444,7 +497,7 @@ __global__ __launch_bounds__(kThreads) void dense_kernel(DenseArgs a) {
       for (int i = 0; i < NACT; ++i) {
         uint4 w4[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) w4[q] = spn[(32 * i + q) * 2];
+        for (int q = 0; q < 4; ++q) w4[q] = spn[(64 * i + q) * 2];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const uint32_t w[3] = {w4[q].x, w4[q].y, w4[q].z};
@@ -466,9 +519,9 @@ __global__ __launch_bounds__(kThreads) void dense_kernel(DenseArgs a) {
             j1 = va > m1 ? static_cast<uint32_t>(j) : j1;
             m1 = __builtin_fmaxf(m1, va);
           }
-          gl1[lw + (32 * i + q) * kEpiRow] = badacc != badacc ? __builtin_nanf("") : m1;
-          gl2[lw + (32 * i + q) * kEpiRow] = m2;
-          glj[lw + (32 * i + q) * kEpiRow] = static_cast<uint8_t>(j1);
+          gl1[lw + (64 * i + q) * kEpiRow] = badacc != badacc ? __builtin_nanf("") : m1;
+          gl2[lw + (64 * i + q) * kEpiRow] = m2;
+          glj[lw + (64 * i + q) * kEpiRow] = static_cast<uint8_t>(j1);
         }
       }
       __syncthreads();
@@ -476,7 +529,7 @@ __global__ __launch_bounds__(kThreads) void dense_kernel(DenseArgs a) {
       // best allowed score, b the bound, L = fl(G - b); the members are the
       // lane bests with fl(g + b) >= L (a lane's other scores are at most its
       // second best: when that qualifies too, the record is crowded)
-      {
+      if (es < kDensePanelSlots) {
         float tn_max = sh.tn[0];
 #pragma unroll
         for (int w = 1; w < kMmaWaves; ++w) {
@@ -485,8 +538,8 @@ __global__ __launch_bounds__(kThreads) void dense_kernel(DenseArgs a) {
         }
         const uint32_t s = es;
         const uint32_t kind = sh.slot_kind[s];
-        const uint4 h0 = sh.span[b][s][0];
-        const uint4 h1 = sh.span[b][s][1];
+        const uint4 h0 = sh.span[s][0];
+        const uint4 h1 = sh.span[s][1];
         const uint32_t lo = h0.w;
         const uint32_t cnt = h1.w;
         TileRecord& rec = stage_rec[s];
@@ -567,10 +620,6 @@ __global__ __launch_bounds__(kThreads) void dense_kernel(DenseArgs a) {
     return;
   }
   switch (nact) {
-    case 8: mfma_tiles.template operator()<8>(); break;
-    case 7: mfma_tiles.template operator()<7>(); break;
-    case 6: mfma_tiles.template operator()<6>(); break;
-    case 5: mfma_tiles.template operator()<5>(); break;
     case 4: mfma_tiles.template operator()<4>(); break;
     case 3: mfma_tiles.template operator()<3>(); break;
     case 2: mfma_tiles.template operator()<2>(); break;
@@ -582,7 +631,7 @@ __global__ __launch_bounds__(kThreads) void dense_kernel(DenseArgs a) {
 }  // namespace
 
 hipError_t launch_dense(const DenseArgs& args, hipStream_t stream) {
-  if (args.H % 32u != 0 || args.H / 32u < static_cast<uint32_t>(kStages) || args.groups < 8u ||
+  if (args.H % 32u != 0 || args.H <= 2u * kKC || args.groups < 8u ||
       args.groups % 8u != 0 || args.z_hi == nullptr || args.spans == nullptr) {
     return hipErrorInvalidValue;
   }
