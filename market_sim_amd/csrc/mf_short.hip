@@ -7,7 +7,7 @@
 // order (greedy.cu:171-176), so every score is exact and no window, bound or
 // record of fast scores is needed.  Wave 0 runs the norm's reference-order
 // chain (operators.cpp:520-534) while waves 1-3 stage the part's candidate
-// rows in LDS (24 pieces of 16 bytes per lane in flight).  The workgroup
+// rows in LDS (8 pieces of 16 bytes per lane in flight).  The workgroup
 // selects by the reference rule (greedy.cu:84-100, 177-211: highest score,
 // lowest id on ties, NaN never wins, an all-NaN row takes its lowest id).
 // With one part the workgroup writes the row's outputs and advances the
@@ -74,7 +74,11 @@ __device__ inline void stage_part(const TailNormArgs& n, const FinalizeArgs& f, 
   }
   wave_sync();
   const uint32_t cnt = m > part ? (m - part + parts - 1u) / parts : 0u;
-  constexpr uint32_t kBatch = 24;
+  // Pieces of a lane in flight.  8 keep the kernel at 68 registers (seven
+  // workgroups per compute unit where LDS allows), 16 and 24 at 114 and 162
+  // (four and three): 1000 rows of lists to 12 at H = 576 take 9.9, 10.0 and
+  // 16.3 us, 64 rows of lists to 256 12.6, 12.5 and 12.9.
+  constexpr uint32_t kBatch = 8;
   const uint32_t per = H / 8u;
   const uint32_t total = cnt * per;
   // piece q = q0 + u kWave of the staged rows is piece q % per of the
@@ -345,8 +349,15 @@ hipError_t launch_short(const TailNormArgs& n, const FinalizeArgs& f, const Shor
                             n.rows > kShortCountRows))) {
     return hipErrorInvalidValue;
   }
+  // LDS for the longest list that a row can have (row_list takes none beyond
+  // max_count), not for all that a part may hold: LDS says how many workgroups
+  // a compute unit runs at once, and a pack of more rows than compute units
+  // runs in that many fewer rounds (1000 rows of lists to 12 at H = 576: 16.3
+  // against 30.8 us, one workgroup at a time).
+  const uint32_t staged =
+      short_stage_rows(n.H, split.per_part < n.max_count ? split.per_part : n.max_count);
   const size_t lds = 3u * static_cast<size_t>(n.H) * sizeof(float) +
-                     static_cast<size_t>(split.per_part) * 2u * (n.H + 8u);
+                     static_cast<size_t>(staged) * 2u * (n.H + 8u);
   hipLaunchKernelGGL(short_tail_kernel, dim3(split.parts, n.rows), dim3(kShortThreads), lds,
                      stream, n, f, split);
   return hipGetLastError();

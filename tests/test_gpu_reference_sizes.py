@@ -156,3 +156,36 @@ def test_head_words_blocks_and_ties(hidden, width):
                                       stream()))
     want, _ = oracle.restricted_output_head_f16(hb, eb, allowed, counts, width)
     assert host(out, np.uint32).tolist() == want.tolist()
+
+
+@pytest.mark.parametrize("order", [0, 1])
+@pytest.mark.parametrize("rows,lists,hidden", [
+    (600, 1, 576), (530, 9, 64), (513, 8, 4096), (700, 33, 1024), (520, 71, 1024), (520, 127, 576),
+    (3, 128, 576)])
+def test_one_kernel_tail_stages_the_longest_list(rows, lists, hidden, order):
+    """Packs of more rows than compute units, one part each: the stage holds
+    exactly the longest list (one row of the table up to all that fit), every
+    second list has it, one row's state lies beyond the table."""
+    from market_sim_amd import workloads as wl
+    from market_sim_amd.tail import DeviceTail
+    w = wl.ragged_pack("short", 11, 3000, hidden, rows, "uniform", lists, 0.0, size_lo=lists)
+    keep = np.ones(w.state_tokens.size, bool)
+    offs = w.state_offsets.astype(np.int64)
+    for s in range(1, w.states, 2):       # shorter by s % lists ids
+        keep[offs[s + 1] - s % lists:offs[s + 1]] = False
+    cut = np.concatenate([[0], np.cumsum(keep)])[offs]
+    w.state_tokens, w.state_offsets = w.state_tokens[keep], cut.astype(np.uint32)
+    if w.state_next is not None:
+        w.state_next = w.state_next[keep]
+    w.row_state = w.row_state.copy()
+    w.row_state[rows // 2] = w.states + 7
+    tail = DeviceTail(w, order=order)
+    assert tail.fused
+    tok, sc, nx = tail.run()
+    etok, esc, enx = oracle.decode_tail(w.x, w.norm_weight, w.epsilon, w.embedding, w.row_state,
+                                        w.state_offsets, w.state_tokens, state_next=w.state_next,
+                                        next_table=w.next_table, order=order, threads=8)
+    nan = np.isnan(esc)
+    assert np.array_equal(tok, etok) and np.array_equal(nx, enx)
+    assert np.array_equal(np.isnan(sc), nan)
+    assert np.array_equal(sc.view(np.uint32)[~nan], esc.view(np.uint32)[~nan])
