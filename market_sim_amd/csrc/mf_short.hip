@@ -7,7 +7,8 @@
 // order (greedy.cu:171-176), so every score is exact and no window, bound or
 // record of fast scores is needed.  Wave 0 runs the norm's reference-order
 // chain (operators.cpp:520-534) while waves 1-3 stage the part's candidate
-// rows in LDS (8 pieces of 16 bytes per lane in flight).  The workgroup
+// rows in LDS (8 pieces of 16 bytes per lane in flight), all at once or, where
+// that lets more workgroups share a compute unit, in rounds.  The workgroup
 // selects by the reference rule (greedy.cu:84-100, 177-211: highest score,
 // lowest id on ties, NaN never wins, an all-NaN row takes its lowest id).
 // With one part the workgroup writes the row's outputs and advances the
@@ -30,6 +31,7 @@ namespace {
 
 constexpr uint32_t kShortWaves = 4;
 constexpr uint32_t kShortThreads = kShortWaves * kWave;
+constexpr uint64_t kShortCUs = 256;  // of an MI355X
 
 // The selection of a list (or part of one): the best candidate, the lowest
 // id and its position (for an all-NaN list), and whether an id lay outside
@@ -75,7 +77,7 @@ __device__ inline void stage_part(const TailNormArgs& n, const FinalizeArgs& f, 
   wave_sync();
   const uint32_t cnt = m > part ? (m - part + parts - 1u) / parts : 0u;
   // Pieces of a lane in flight.  8 keep the kernel at 68 registers (seven
-  // workgroups per compute unit where LDS allows), 16 and 24 at 114 and 162
+  // workgroups per compute unit where LDS allows; 95 and five in rounds), 16 and 24 at 114 and 162
   // (four and three): 1000 rows of lists to 12 at H = 576 take 9.9, 10.0 and
   // 16.3 us, 64 rows of lists to 256 12.6, 12.5 and 12.9.
   constexpr uint32_t kBatch = 8;
@@ -164,8 +166,11 @@ __device__ inline void short_finish(const TailNormArgs& n, const FinalizeArgs& f
   if (slot != nullptr) *slot = next;
 }
 
+// kRounds: a list may be longer than `stage`, the rows staged at once (a kernel
+// of its own: the loop costs a single round 2%).
+template <bool kRounds>
 __global__ __launch_bounds__(kShortThreads) void short_tail_kernel(TailNormArgs n, FinalizeArgs f,
-                                                                   ShortSplit split) {
+                                                                   ShortSplit split, uint32_t stage) {
   extern __shared__ __align__(16) float lds[];
   __shared__ ShortShared sh;
   const uint32_t H = n.H;
@@ -223,47 +228,56 @@ __global__ __launch_bounds__(kShortThreads) void short_tail_kernel(TailNormArgs 
   // this part's candidates: list positions base .. base + m - 1
   const uint32_t base = part * split.per_part;
   const uint32_t m = count - base < split.per_part ? count - base : split.per_part;
-  if (wave == 0) {
-    const float sum_squares = weighted ? sequential_sum_wave(sq, H) : 0.0f;
-    if (lane == 0) sh.inv = weighted ? norm_inverse(sum_squares, H, n.epsilon) : 1.0f;
-  } else {
-    stage_part(n, f, sh, es, base, m, wave - 1u, kShortWaves - 1u);
-  }
-  __syncthreads();
-  // y = (x * inv) * w in the reference's roundings (operators.cpp:533-534)
-  const float inv = sh.inv;
-  if (weighted) {
-    for (uint32_t c = tid; c < H; c += kShortThreads) xs[c] = (xs[c] * inv) * ws[c];
-  }
-  __syncthreads();
-
   Best best = best_identity();
   uint32_t mt = kInvalidToken;
   uint32_t mp = 0u;
-  if (tid < m) {
-    const uint32_t token = sh.cand[tid];
-    const uint32_t pos = base + tid;
-    if (token >= n.V) {
-      sh.invalid = 1u;
+  uint32_t j0 = 0u;
+  do {
+    const uint32_t mj = kRounds && m - j0 > stage ? stage : m - j0;
+    // wave 0 has the norm's chain in the first round and helps from then on
+    const uint32_t busy = j0 == 0u ? 1u : 0u;
+    if (j0 != 0u) __syncthreads();  // the round before is scored: its rows are free
+    if (wave < busy) {
+      const float sum_squares = weighted ? sequential_sum_wave(sq, H) : 0.0f;
+      if (lane == 0) sh.inv = weighted ? norm_inverse(sum_squares, H, n.epsilon) : 1.0f;
     } else {
-      // the candidate's next state, loaded under the chain (greedy.cu
-      // leaves the advance to the caller; operators.cpp steps the DFA)
-      uint32_t nx = kInvalidToken;
-      if (f.state_next != nullptr) {
-        nx = f.state_next[meta.list_begin + pos];
-      } else if (f.next_table != nullptr) {
-        nx = static_cast<uint32_t>(f.next_table[static_cast<uint64_t>(meta.state) * f.V + token]);
-      }
-      __builtin_amdgcn_sched_barrier(0);  // the load goes out before the chain
-      const uint32_t rs = H + 8u;
-      const float s = f.order == 1 ? chain_lds<true>(xs, es + tid * rs, H)
-                                   : chain_lds<false>(xs, es + tid * rs, H);
-      best = best_leaf(s, token, pos);
-      mt = token;
-      mp = pos;
-      sh.nx[tid] = nx;
+      stage_part(n, f, sh, es, base + j0, mj, wave - busy, kShortWaves - busy);
     }
-  }
+    if (j0 == 0u && weighted) {
+      __syncthreads();
+      // y = (x * inv) * w in the reference's roundings (operators.cpp:533-534)
+      const float inv = sh.inv;
+      for (uint32_t c = tid; c < H; c += kShortThreads) xs[c] = (xs[c] * inv) * ws[c];
+    }
+    __syncthreads();
+    if (tid < mj) {
+      const uint32_t token = sh.cand[tid];
+      const uint32_t pos = base + j0 + tid;
+      if (token >= n.V) {
+        sh.invalid = 1u;
+      } else {
+        // the candidate's next state, loaded under the chain (greedy.cu
+        // leaves the advance to the caller; operators.cpp steps the DFA)
+        uint32_t nx = kInvalidToken;
+        if (f.state_next != nullptr) {
+          nx = f.state_next[meta.list_begin + pos];
+        } else if (f.next_table != nullptr) {
+          nx = static_cast<uint32_t>(f.next_table[static_cast<uint64_t>(meta.state) * f.V + token]);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // the load goes out before the chain
+        const uint32_t rs = H + 8u;
+        const float s = f.order == 1 ? chain_lds<true>(xs, es + tid * rs, H)
+                                     : chain_lds<false>(xs, es + tid * rs, H);
+        best = best_of(best, best_leaf(s, token, pos));
+        if (token < mt || (token == mt && pos < mp)) {
+          mt = token;
+          mp = pos;
+        }
+        sh.nx[j0 + tid] = nx;
+      }
+    }
+    j0 += mj;
+  } while (kRounds && j0 < m);
   best = wave_best(best);
   wave_min_token(mt, mp);
   if (lane == 0) {
@@ -339,6 +353,41 @@ uint32_t short_stage_rows(uint32_t H, uint32_t max_count) {
   return static_cast<uint32_t>(rows < want ? rows : want);
 }
 
+namespace {
+
+// Rows that one round stages.  A workgroup whose list is longer stages and
+// scores it in rounds, so that more workgroups share a compute unit's LDS.
+// With k of them at once the launch runs in ceil(groups / 256 k) turns, each a
+// start (the list, x, the norm's chain) and the rounds of the longest list; a
+// round takes about twice a start, and the cheapest k is taken.  Measured at
+// H = 576, one round against this: 500 rows of lists to 100 23.8 and 17.0 us,
+// 700 to 50 17.8 and 15.0, 1000 to 100 43.0 and 26.0; H = 1024, 300 to 64 26.1
+// and 20.6, 700 to 64 40.2 and 34.4; H = 2048, 1000 to 16 80.1 and 64.1.  700 to
+// 30 at H = 2048 stay in one round (58.9; five rounds 72.1).
+uint32_t short_round(uint32_t H, uint32_t most, uint64_t groups) {
+  constexpr uint64_t kLds = 160u * 1024u;  // of a compute unit, given out in 1280-byte pieces
+  constexpr uint64_t kPiece = 1280u;
+  constexpr uint32_t kFit = 5;             // workgroups that 96 registers allow
+  const uint64_t fixed = sizeof(ShortShared) + 12ull * H;
+  uint32_t stage = most;
+  uint64_t least = ~0ull;
+  for (uint64_t k = 1; k <= kFit; ++k) {
+    const uint64_t share = kLds / k / kPiece * kPiece;
+    const uint64_t fits = share > fixed ? (share - fixed) / (2ull * (H + 8u)) : 0u;
+    if (fits == 0u) break;
+    const uint32_t rows = fits < most ? static_cast<uint32_t>(fits) : most;
+    const uint64_t turns = (groups + kShortCUs * k - 1u) / (kShortCUs * k);
+    const uint64_t cost = turns * (1u + 2u * ((most + rows - 1u) / rows));
+    if (cost <= least) {
+      least = cost;
+      stage = rows;
+    }
+  }
+  return stage;
+}
+
+}  // namespace
+
 hipError_t launch_short(const TailNormArgs& n, const FinalizeArgs& f, const ShortSplit& split,
                         hipStream_t stream) {
   const uint32_t stage_rows = short_stage_rows(n.H, split.per_part);
@@ -352,14 +401,16 @@ hipError_t launch_short(const TailNormArgs& n, const FinalizeArgs& f, const Shor
   // LDS for the longest list that a row can have (row_list takes none beyond
   // max_count), not for all that a part may hold: LDS says how many workgroups
   // a compute unit runs at once, and a pack of more rows than compute units
-  // runs in that many fewer rounds (1000 rows of lists to 12 at H = 576: 16.3
+  // runs in that many fewer turns (1000 rows of lists to 12 at H = 576: 9.9
   // against 30.8 us, one workgroup at a time).
-  const uint32_t staged =
+  const uint32_t most =
       short_stage_rows(n.H, split.per_part < n.max_count ? split.per_part : n.max_count);
+  const uint32_t stage = short_round(n.H, most, static_cast<uint64_t>(split.parts) * n.rows);
   const size_t lds = 3u * static_cast<size_t>(n.H) * sizeof(float) +
-                     static_cast<size_t>(staged) * 2u * (n.H + 8u);
-  hipLaunchKernelGGL(short_tail_kernel, dim3(split.parts, n.rows), dim3(kShortThreads), lds,
-                     stream, n, f, split);
+                     static_cast<size_t>(stage) * 2u * (n.H + 8u);
+  const auto kernel = stage < most ? short_tail_kernel<true> : short_tail_kernel<false>;
+  hipLaunchKernelGGL(kernel, dim3(split.parts, n.rows), dim3(kShortThreads), lds, stream, n, f,
+                     split, stage);
   return hipGetLastError();
 }
 

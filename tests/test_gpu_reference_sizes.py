@@ -161,11 +161,13 @@ def test_head_words_blocks_and_ties(hidden, width):
 @pytest.mark.parametrize("order", [0, 1])
 @pytest.mark.parametrize("rows,lists,hidden", [
     (600, 1, 576), (530, 9, 64), (513, 8, 4096), (700, 33, 1024), (520, 71, 1024), (520, 127, 576),
-    (3, 128, 576)])
+    (3, 128, 576), (700, 50, 576), (500, 100, 576), (250, 128, 576), (1030, 16, 2048)])
 def test_one_kernel_tail_stages_the_longest_list(rows, lists, hidden, order):
-    """Packs of more rows than compute units, one part each: the stage holds
-    exactly the longest list (one row of the table up to all that fit), every
-    second list has it, one row's state lies beyond the table."""
+    """Packs of more rows than compute units, one part or two: the stage holds
+    exactly the longest list (one row of the table up to all that fit) or a
+    share of it, in two rounds and more.  Every second list is the longest; one
+    row's state lies beyond the table, one list ends in an id outside the
+    vocabulary, one row is all NaN."""
     from market_sim_amd import workloads as wl
     from market_sim_amd.tail import DeviceTail
     w = wl.ragged_pack("short", 11, 3000, hidden, rows, "uniform", lists, 0.0, size_lo=lists)
@@ -179,9 +181,14 @@ def test_one_kernel_tail_stages_the_longest_list(rows, lists, hidden, order):
         w.state_next = w.state_next[keep]
     w.row_state = w.row_state.copy()
     w.row_state[rows // 2] = w.states + 7
+    w.state_tokens = w.state_tokens.copy()
+    w.state_tokens[w.state_offsets[w.row_state[0] + 1] - 1] = w.vocab
+    w.x = w.x.copy()
+    w.x[2] = np.nan
     tail = DeviceTail(w, order=order)
     assert tail.fused
     tok, sc, nx = tail.run()
+    assert tok[0] == tok[rows // 2] == 0xFFFFFFFF and np.isnan(sc[2])
     etok, esc, enx = oracle.decode_tail(w.x, w.norm_weight, w.epsilon, w.embedding, w.row_state,
                                         w.state_offsets, w.state_tokens, state_next=w.state_next,
                                         next_table=w.next_table, order=order, threads=8)
