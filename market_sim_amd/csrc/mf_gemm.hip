@@ -8,9 +8,9 @@
 // launch_projection).  Eight MFMA waves, two a SIMD, each multiply 64 rows x
 // kNT / 2 tokens as 4 x kNT / 32 blocks of v_mfma_f32_16x16x32_f16, so one
 // wave's MFMAs run under the other's LDS reads.  The tokens are the first
-// operand: a lane then holds consecutive tokens of one row, and with the
-// token rows of a block pair interleaved (token_row) eight of them, which it
-// stores as 16 bytes straight from its registers.
+// operand: a lane then holds four consecutive tokens of one row, or, for FP16
+// results, with the token rows of a block pair interleaved (token_row), eight,
+// which it stores as 16 bytes straight from its registers.
 //
 // K runs in chunks of 64 features (whole 128-byte lines).  A chunk's A rows
 // and E rows go straight from memory into LDS by global_load_lds copies.  Four
@@ -79,12 +79,22 @@ constexpr uint32_t kGemmLds = Ring<kMT>::kSlots * Ring<kMT>::kBytes + Ring<kNT>:
 static_assert(kGemmLds<192> <= 160u * 1024u, "LDS");
 
 // The piece p of A row r sits at p ^ a_swz(r), of E row t at p ^ b_swz(t).
-// A fragment reads 16 consecutive A rows, or E rows 8 i + {0..3} (+ 4).
+// A fragment reads 16 consecutive A rows, or, where the result is FP16 (kPair),
+// E rows 8 i + {0..3} (+ 4), else 16 consecutive ones as well.
 __device__ __forceinline__ uint32_t a_swz(uint32_t r) { return (r >> 1) & 7u; }
-__device__ __forceinline__ uint32_t b_swz(uint32_t t) { return ((t >> 1) & 1u) | ((t >> 2) & 6u); }
-// Token (of 32) that row i of block 0 or 1 of a pair holds.
+template <bool kPair>
+__device__ __forceinline__ uint32_t b_swz(uint32_t t) {
+  return kPair ? ((t >> 1) & 1u) | ((t >> 2) & 6u) : (t >> 1) & 7u;
+}
+// Token (of 32) that row i of block 0 or 1 of a pair holds.  A lane's results
+// are 16 bytes of consecutive tokens either way: eight FP16 of a block pair,
+// or four FP32 of each block.  One store instruction then fills whole 64-byte
+// pieces of a row.  With pairs for FP32 too, every store left half of each
+// 32 bytes to the next one: the product of 256 x 576 x 49152, written through,
+// took 59 us, and the comparator's step around it 86 instead of 53.
+template <bool kPair>
 __device__ __forceinline__ uint32_t token_row(uint32_t block, uint32_t i) {
-  return 8u * (i / 4u) + 4u * block + i % 4u;
+  return kPair ? 8u * (i / 4u) + 4u * block + i % 4u : 16u * block + i;
 }
 
 // Wait until at most kN of this wave's vector memory operations are in flight.
@@ -100,9 +110,11 @@ __device__ __forceinline__ void chunk_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// Results of tiles of few chunks are written through to memory (whole rows of
-// 16-byte words only): the workgroups' stores then come close together, and
-// what stays dirty in L2 is written back after the last of them.
+// FP16 results of tiles of few chunks are written through to memory (whole rows
+// of 16-byte words only): the workgroups' stores then come close together, and
+// what stays dirty in L2 is written back after the last of them.  FP32 scores
+// are read by the selection that follows (comparator of 256 rows at H = 576,
+// V = 49152: 53.3 us, written through 54.6).
 constexpr uint32_t kThroughChunks = 15;
 
 // 16 bytes to global memory at any element (gfx950 stores need no alignment).
@@ -190,7 +202,7 @@ __global__ __launch_bounds__(kThreads) void projection_kernel(ProjArgs a, uint32
       for (uint32_t i = 0; i < RB::kCopies; ++i) {
         const uint32_t t = cr + 8u * kCopyWaves * i;
         const uint32_t tok = n0 + t < a.V ? n0 + t : a.V - 1u;
-        burst_to_lds(a.emb + static_cast<uint64_t>(tok) * a.H + feature(sb.c, (lane % 8u) ^ b_swz(t)),
+        burst_to_lds(a.emb + static_cast<uint64_t>(tok) * a.H + feature(sb.c, (lane % 8u) ^ b_swz<kF16Out>(t)),
                      buf + (cw + kCopyWaves * i) * 1024u);
       }
       advance(sb, RB::kUnits, RB::kSlots);
@@ -273,8 +285,8 @@ __global__ __launch_bounds__(kThreads) void projection_kernel(ProjArgs a, uint32
     }
 #pragma unroll
     for (uint32_t i = 0; i < kTB; ++i) {
-      const uint32_t t = br + 32u * (i / 2u) + token_row(i % 2u, col);
-      f.b[i] = *reinterpret_cast<const half8_t*>(bbuf + t * kRow + (p ^ b_swz(t)) * 16u);
+      const uint32_t t = br + 32u * (i / 2u) + token_row<kF16Out>(i % 2u, col);
+      f.b[i] = *reinterpret_cast<const half8_t*>(bbuf + t * kRow + (p ^ b_swz<kF16Out>(t)) * 16u);
     }
   };
   bool norms = false;
@@ -301,7 +313,7 @@ __global__ __launch_bounds__(kThreads) void projection_kernel(ProjArgs a, uint32
   };
 
   chunk_barrier();
-  const bool through = chunks <= kThroughChunks && a.V % 8u == 0u;
+  const bool through = kF16Out && chunks <= kThroughChunks && a.V % 8u == 0u;
   uint32_t c = 0, j_tile = idx;
   for (uint32_t q = 0; q < total; ++q) {
     norms = !kF16Out && a.tok_norm != nullptr && wm == 0u && j_tile % m_tiles == 0u;
@@ -330,21 +342,23 @@ __global__ __launch_bounds__(kThreads) void projection_kernel(ProjArgs a, uint32
           float sq = tok_sq[i];
           sq += __shfl_xor(sq, 16);
           sq += __shfl_xor(sq, 32);
-          const uint32_t tok = n0 + 32u * (i / 2u) + token_row(i % 2u, ecol);
+          const uint32_t tok = n0 + 32u * (i / 2u) + token_row<kF16Out>(i % 2u, ecol);
           if (ekb == 0u && tok < a.V) a.tok_norm[tok] = __fsqrt_rn(sq) * (1.0f + 0x1p-7f);
         }
       }
     }
+    constexpr uint32_t kLaneBlocks = kF16Out ? 2u : 1u;
+    constexpr uint32_t kLaneTokens = 4u * kLaneBlocks;
     auto store = [&]<bool kThrough>() {
 #pragma unroll
       for (uint32_t j = 0; j < kRB; ++j) {
         const uint32_t row = m0 + 16u * j + ecol;
         const uint64_t at = static_cast<uint64_t>(row) * a.V;
 #pragma unroll
-        for (uint32_t i = 0; i < kTB; i += 2u) {
-          const uint32_t tok = n0 + 16u * i + 8u * ekb;  // this lane's eight tokens
+        for (uint32_t i = 0; i < kTB; i += kLaneBlocks) {
+          const uint32_t tok = n0 + 16u * i + kLaneTokens * ekb;  // this lane's tokens
           if (row >= a.m || tok >= a.V) continue;
-          if (a.V - tok >= 8u) {  // (16-byte stores at any element: rows of odd V too)
+          if (a.V - tok >= kLaneTokens) {  // (16-byte stores at any element: rows of odd V too)
             if constexpr (kF16Out) {
               u32x4 v;
 #pragma unroll
@@ -356,12 +370,11 @@ __global__ __launch_bounds__(kThreads) void projection_kernel(ProjArgs a, uint32
               store16<kThrough>(a.out_f16 + at + tok, v);
             } else {
               store16<kThrough>(a.out_f32 + at + tok, __builtin_bit_cast(u32x4, acc[i][j]));
-              store16<kThrough>(a.out_f32 + at + tok + 4u, __builtin_bit_cast(u32x4, acc[i + 1u][j]));
             }
           } else {
 #pragma unroll
-            for (uint32_t e = 0; e < 8u; ++e) {
-              const float s = e < 4u ? acc[i][j][e % 4u] : acc[i + 1u][j][e % 4u];
+            for (uint32_t e = 0; e < kLaneTokens; ++e) {
+              const float s = acc[i + e / 4u][j][e % 4u];
               if (tok + e < a.V) {
                 if constexpr (kF16Out) {
                   a.out_f16[at + tok + e] = float_to_half_rne(s);

@@ -196,3 +196,19 @@ def test_one_kernel_tail_stages_the_longest_list(rows, lists, hidden, order):
     assert np.array_equal(tok, etok) and np.array_equal(nx, enx)
     assert np.array_equal(np.isnan(sc), nan)
     assert np.array_equal(sc.view(np.uint32)[~nan], esc.view(np.uint32)[~nan])
+
+
+@pytest.mark.parametrize("rows,vocab,hidden", [
+    (3, 17, 64), (65, 203, 64), (130, 4099, 576), (257, 1026, 640), (9, 8193, 1088)])
+def test_full_comparator_scores_at_row_ends(rows, vocab, hidden):
+    """The FP32 projection under the full-vocabulary comparator: rows that end
+    inside a lane's four tokens, in a block and in a tile; one M-tile and two;
+    half a chunk at the end of K."""
+    from market_sim_amd import workloads as wl
+    from market_sim_amd.tail import DeviceTail
+    w = wl.ragged_pack("full", 7, vocab, hidden, rows, "uniform", max(1, vocab // 3), 0.4)
+    tok, sc, nx = DeviceTail(w, full=True).run()
+    etok, esc, enx = oracle.decode_tail(w.x, w.norm_weight, w.epsilon, w.embedding, w.row_state,
+                                        w.state_offsets, w.state_tokens, threads=8)
+    assert np.array_equal(tok, etok) and np.array_equal(nx, enx)
+    assert np.array_equal(sc.view(np.uint32), esc.view(np.uint32))
