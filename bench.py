@@ -268,7 +268,7 @@ def fallback_summary(alg: dict, fb_ms) -> dict:
     bytes by an empty launch)."""
     if alg["B_u"] == 0 or fb_ms is None:
         return {"kernel": "none (no unrestricted rows)", "rows": 0}
-    return {"kernel": "vocab_head_kernel (MFMA head, unrestricted rows)", "rows": alg["B_u"],
+    return {"kernel": "stream_kernel (MFMA head, unrestricted rows)", "rows": alg["B_u"],
             "avg_launch_us": round(fb_ms * 1e3, 2),
             "hbm_GBs": round(alg["fallback_bytes"] / (fb_ms * 1e-3) / 1e9, 1),
             "hbm_frac": round(alg["fallback_bytes"] / (fb_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
